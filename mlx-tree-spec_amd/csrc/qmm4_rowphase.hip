@@ -23,7 +23,7 @@
 //    bf16_rne(fp32(s) * q + fp32(b)); a phase holding a scale outside its range takes
 //    dequant_word). The A operand, lane (m, g), is x[m] at the same 8 k; it is read from LDS once
 //    per (v, t) and feeds the MFMAs of all of the wave's blocks.
-//  * The next phase's x slice (A-fragment order) and the scales and biases of the range's rows are
+//  * The next phase's x slice (row by row) and the scales and biases of the range's rows are
 //    staged in LDS (double-buffered) by the whole workgroup, behind the weight prefetch; one
 //    barrier per phase publishes them.
 //  * Nothing waits for a load before it is needed: the phase barrier is a bare s_barrier behind
@@ -158,24 +158,35 @@ void rowphase_kernel(RowPhaseParams P) {
   uint8_t* const ws_b = ws_s + C::kWinBytes;            // bias window
 
   // ---- staging of one phase's x pieces, global -> LDS directly (no registers) ----
-  // x piece i = (v * 16 + g4 * 4 + t) * MP + m holds x[m][PH ph + 128 v + 32 g4 + 8 t .. + 8):
-  // the A fragment of MFMA (v, t) for lane (m, g4). Rows m >= M read as zero. Wave w's j-th load
-  // fills pieces j * kRpThreads + 64 w .. + 63, one contiguous kilobyte of the stage (the LDS
-  // destination of a lane is the instruction's base + 16 lane). Completion is waited for with an
-  // explicit vector memory count one phase later, before the barrier that publishes the stage.
-  static_assert(C::kXPieces % kRpThreads == 0, "whole x loads per thread");
+  // Row-major: slot m * 16 V + c of the stage holds the 16-byte piece c ^ (m % 16) of row m's run of
+  // PH values (x[m][PH ph + 8 (c ^ (m % 16)) .. + 8)); rows m >= M lie past the resource and read as
+  // zero. Adjacent lanes thus
+  // read adjacent pieces of one row: the address unit merges the lanes of a load only where
+  // neighbouring lanes fall in one 64-byte segment (measured per CU on 1 KB loads that hit L2: 37
+  // GB/s with 16 rows spread over neighbouring lanes, 86 GB/s with 4 or more lanes per row; into LDS
+  // 29 and 64 GB/s). The pieces used to lie in A-fragment order, one row per neighbouring lane; so
+  // (A/B, identical bits) 64 / 32 x 17408 -> 5120 31.8 / 25.0 -> 28.6 / 23.4 us, 112 x 5120 -> 17408
+  // 45.5 -> 38.4, 64 rows of the fused 5120 -> 34816 58.3 -> 47.1, 32 x 5120 -> 151936 (x is a sixth
+  // of its requests) within the spread. The XOR spreads the 16 rows that one fragment read touches
+  // (one piece each at the same place) over all banks. Wave w's j-th load fills slots j *
+  // kRpThreads + 64 w .. + 63, one contiguous kilobyte of the stage (the LDS destination of a lane
+  // is the instruction's base + 16 lane). Completion is waited for with an explicit vector memory count one phase later, before
+  // the barrier that publishes the stage.
+  constexpr int kXC = 16 * V;                // pieces per row and phase
+  constexpr int kXRows = kRpThreads / kXC;   // rows per load of the whole workgroup: 16 or 8
+  static_assert(C::kXPieces % kRpThreads == 0 && (kXRows == 16 || kXRows == 8), "whole x loads per thread");
   typedef __attribute__((address_space(3))) void* lds_ptr;
+  const int xm = tid / kXC;
+  const uint32_t xo = ((uint32_t)xm * (uint32_t)P.K + (uint32_t)(8 * ((tid % kXC) ^ xm))) * 2u;
   auto stage_x = [&](int st, int ph, bool live) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < C::kXL; ++j) {
-      const int i = tid + j * kRpThreads;
-      const int m = i % MP, q = i / MP;  // q = v * 16 + g4 * 4 + t
-      const int v = q >> 4, g4 = (q >> 2) & 3, t = q & 3;
-      const uint32_t off = (live && m < P.M)
-                               ? ((uint32_t)m * (uint32_t)P.K + (uint32_t)(ph * C::PH + 128 * v + 32 * g4 + 8 * t)) * 2u
-                               : kOut;
+      // Row xm + kXRows j: its offset is scalar, and so is its XOR where kXRows = 8 leaves bit 3 of
+      // the row to j (K % 512 == 0 and a phase is 512 or 1024 bytes, so bit 7 of the offset is c's).
+      const uint32_t off = live ? xo ^ (uint32_t)((j * kXRows & 8) * 16) : kOut;
       const lds_ptr dst = (lds_ptr)(reinterpret_cast<uint8_t*>(xs(st)) + (size_t)(j * kRpThreads + 64 * wave) * 16);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, dst, 16, off, 0, 0, 0);
+      const int so = ph * C::PH * 2 + j * kXRows * P.K * 2;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, dst, 16, off, so, 0, 0);
     }
   };
 
@@ -272,7 +283,7 @@ void rowphase_kernel(RowPhaseParams P) {
     for (int t = 0; t < 4; ++t) {
       u32x4 a[MB];
 #pragma unroll
-      for (int i = 0; i < MB; ++i) a[i] = xb[(v * 16 + g * 4 + t) * MP + i * 16 + n];
+      for (int i = 0; i < MB; ++i) a[i] = xb[(i * 16 + n) * kXC + v * 16 + ((g * 4 + t) ^ n)];
       // Blocks past this wave's count hold zero weights (their loads lie outside the buffer)
       // and sums that are never stored: computing them keeps the loop free of branches, except
       // for the last slot of an OPT variant, which only the waves holding a BPW-th block run.
