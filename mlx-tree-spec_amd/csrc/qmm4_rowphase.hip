@@ -160,18 +160,17 @@ void rowphase_kernel(RowPhaseParams P) {
   // ---- staging of one phase's x pieces, global -> LDS directly (no registers) ----
   // Row-major: slot m * 16 V + c of the stage holds the 16-byte piece c ^ (m % 16) of row m's run of
   // PH values (x[m][PH ph + 8 (c ^ (m % 16)) .. + 8)); rows m >= M lie past the resource and read as
-  // zero. Adjacent lanes thus
-  // read adjacent pieces of one row: the address unit merges the lanes of a load only where
-  // neighbouring lanes fall in one 64-byte segment (measured per CU on 1 KB loads that hit L2: 37
-  // GB/s with 16 rows spread over neighbouring lanes, 86 GB/s with 4 or more lanes per row; into LDS
-  // 29 and 64 GB/s). The pieces used to lie in A-fragment order, one row per neighbouring lane; so
-  // (A/B, identical bits) 64 / 32 x 17408 -> 5120 31.8 / 25.0 -> 28.6 / 23.4 us, 112 x 5120 -> 17408
-  // 45.5 -> 38.4, 64 rows of the fused 5120 -> 34816 58.3 -> 47.1, 32 x 5120 -> 151936 (x is a sixth
-  // of its requests) within the spread. The XOR spreads the 16 rows that one fragment read touches
-  // (one piece each at the same place) over all banks. Wave w's j-th load fills slots j *
-  // kRpThreads + 64 w .. + 63, one contiguous kilobyte of the stage (the LDS destination of a lane
-  // is the instruction's base + 16 lane). Completion is waited for with an explicit vector memory count one phase later, before
-  // the barrier that publishes the stage.
+  // zero. Adjacent lanes thus read adjacent pieces of one row: the address unit merges the lanes of
+  // a load only where neighbouring lanes fall in one 64-byte segment (measured per CU on 1 KB loads
+  // that hit L2: 37 GB/s with 16 rows spread over neighbouring lanes, 86 GB/s with 4 or more lanes
+  // per row; into LDS 29 and 64 GB/s). The pieces used to lie in A-fragment order, one row per
+  // neighbouring lane; so (A/B, identical bits) 64 / 32 x 17408 -> 5120 31.8 / 25.0 -> 28.6 / 23.4 us,
+  // 112 x 5120 -> 17408 45.5 -> 38.4, 64 rows of the fused 5120 -> 34816 58.3 -> 47.1, 32 x 5120 ->
+  // 151936 (x is a sixth of its requests) within the spread. The XOR spreads the 16 rows that one
+  // fragment read touches (one piece each at the same place) over all banks. Wave w's j-th load
+  // fills slots j * kRpThreads + 64 w .. + 63, one contiguous kilobyte of the stage (the LDS
+  // destination of a lane is the instruction's base + 16 lane). Completion is waited for with an
+  // explicit vector memory count one phase later, before the barrier that publishes the stage.
   constexpr int kXC = 16 * V;                // pieces per row and phase
   constexpr int kXRows = kRpThreads / kXC;   // rows per load of the whole workgroup: 16 or 8
   static_assert(C::kXPieces % kRpThreads == 0 && (kXRows == 16 || kXRows == 8), "whole x loads per thread");

@@ -110,6 +110,9 @@ struct Scales {
   uint32_t d[V];  // the 2V bf16 scales (or biases) of one row for one unit
 };
 
+// (Loading a unit's scales merged, four lanes per row and a dword each, and putting them back in
+// MFMA order through the wave's LDS, as the 9-16-row form below does, was 5-12% slower at 1-4 rows:
+// the LDS round trip at the head of every unit costs more than the merged loads save.)
 template <int V>
 __device__ __forceinline__ Scales<V> load_scales(__amdgpu_buffer_rsrc_t r, uint32_t voff, int soff) {
   Scales<V> o;
@@ -125,8 +128,12 @@ __device__ __forceinline__ Scales<V> load_scales(__amdgpu_buffer_rsrc_t r, uint3
   return o;
 }
 
-// Dynamic LDS: x pieces [S][16][MP] (A-fragment order), unit slots [U][MP / 4][16] f32x4, a spare
-// 16-byte slot (the target of surplus x pieces, so that every x store is unconditional), the counter.
+// Data that a wave's lanes hand to each other through the wave's own LDS needs no barrier (a wave's
+// LDS accesses complete in order), but the compiler, which sees one lane, must keep the order too.
+__device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
+
+// Dynamic LDS: x pieces [16 S][MP] or [MP][16 S] (see the staging), unit slots [U][MP / 4][16] f32x4, a spare 16-byte slot (the target of surplus x pieces, so that every x store
+// is unconditional), the counter.
 __host__ __device__ inline size_t rowsplit_xs_bytes(int K, int MP) { return (size_t)(K >> 7) * 16 * MP * 16; }
 __host__ __device__ inline size_t rowsplit_part_bytes(int units, int MP) { return (size_t)units * (MP / 4) * 16 * 16; }
 
@@ -185,49 +192,83 @@ void rowsplit_kernel(RowSplitParams P) {
   const int r1 = min(P.Nout, r0 + P.R);
   const int KG = P.K >> 6;
 
-  // x pieces: item i = sq * M + m is the 16-byte piece sq (k = 8 sq .. 8 sq + 7) of row m, stored
-  // at LDS position sq * MP + m. All batches but the last are staged before any weight fetch;
-  // the last batch is loaded before the first fetches and stored after them. Loads past the last
-  // item go to an offset outside the buffer resource (zeros, no memory access); the stores are
-  // unconditional (surplus pieces go to the spare slot): a store under a branch would let the
-  // compiler move its load there, behind the fetches, and wait for all of them.
-  const int xitems = S * 16 * P.M;
+  // x pieces: an item is the 16-byte piece sq (k = 8 sq .. 8 sq + 7) of row m. More than 4 rows
+  // (MERGE): items row by row (L = 16 S pieces per row), so that neighbouring lanes load neighbouring
+  // pieces, which the address unit merges (it takes 16 rows spread over neighbouring lanes at less
+  // than half that rate); stored at A-fragment position sq * MP + (m ^ (sq / 4) % 4), the XOR
+  // spreading the pieces of one store over the banks: 13-16 x 5120 -> 17408 and 5 x 5120 -> 12288
+  // 20.4-20.8 / 13.0 -> 20.0-20.2 / 12.6 us. Up to 4 rows: item i = sq * M + m at position sq * MP + m
+  // (the row-by-row walk's longer prologue cost 1 x 5120 -> 5120 7.8 -> 8.0 us). All batches but the
+  // last are staged before any weight fetch; the last batch is loaded before the first fetches and
+  // stored after them. Loads past the last item go to an offset outside the buffer resource (zeros,
+  // no memory access); the stores are unconditional (surplus pieces go to the spare slot): a store
+  // under a branch would let the compiler move its load there, behind the fetches, and wait for all
+  // of them.
+  constexpr bool ROWX = SMALL || OWN;   // x row by row in LDS, by DMA
+  constexpr bool MERGE = MP > 4 && !ROWX;
+  const int L = S * 16;
+  const int xitems = L * P.M;
   const int nxb = (xitems + kRsThreads * kRsXB - 1) / (kRsThreads * kRsXB);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(P.x), 0, rsrc_bytes((unsigned long long)P.M * P.K * 2), kBufferRsrcWord3);
   u32x4 xr[kRsXB];
+  int xp[kRsXB];  // MERGE: the LDS position of each item held in xr
+  // MERGE: row and piece of this thread's next item (items tid, tid + kRsThreads, ... in turn).
+  int xm = 0, xq = 0, xdm = 0, xdq = 0;
+  if constexpr (MERGE) {
+    xm = tid / L;
+    xq = tid - xm * L;
+    xdm = kRsThreads / L;
+    xdq = kRsThreads - xdm * L;
+  }
   auto load_x = [&](int batch) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < kRsXB; ++j) {
-      const int i = tid + (batch * kRsXB + j) * kRsThreads;
-      const int sq = i / P.M, m = i - sq * P.M;
-      const uint32_t off =
-          i < xitems ? ((uint32_t)m * (uint32_t)P.K + (uint32_t)kq + (uint32_t)sq * 8u) * 2u : 0x80000000u;
+      uint32_t off;
+      if constexpr (MERGE) {
+        xp[j] = xm < P.M ? xq * MP + (xm ^ ((xq >> 2) & 3)) : (int)(spare - xs);
+        off = xm < P.M ? ((uint32_t)xm * (uint32_t)P.K + (uint32_t)kq + (uint32_t)xq * 8u) * 2u : 0x80000000u;
+        xm += xdm;
+        xq += xdq;
+        if (xq >= L) {
+          xq -= L;
+          ++xm;
+        }
+      } else {
+        const int i = tid + (batch * kRsXB + j) * kRsThreads;
+        const int sq = i / P.M, m = i - sq * P.M;
+        off = i < xitems ? ((uint32_t)m * (uint32_t)P.K + (uint32_t)kq + (uint32_t)sq * 8u) * 2u : 0x80000000u;
+      }
       xr[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0);
     }
   };
   auto store_x = [&](int batch) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < kRsXB; ++j) {
-      const int i = tid + (batch * kRsXB + j) * kRsThreads;
-      const int sq = i / P.M, m = i - sq * P.M;
-      u32x4* dst = i < xitems ? xs + (sq * MP + m) : spare;
-      *dst = xr[j];
+      if constexpr (MERGE) {
+        xs[xp[j]] = xr[j];
+      } else {
+        const int i = tid + (batch * kRsXB + j) * kRsThreads;
+        const int sq = i / P.M, m = i - sq * P.M;
+        u32x4* dst = i < xitems ? xs + (sq * MP + m) : spare;
+        *dst = xr[j];
+      }
     }
   };
-  // SMALL: x straight into LDS (buffer loads with the LDS bit): LDS slot q = sq * MP + m holds
-  // piece sq of row m, rows m >= M read as zero. A wave's instruction fills 64 consecutive slots
-  // (the instruction's base + 16 lane); the slot count S * 16 * MP is a multiple of 64, so a wave
+  // ROWX: x straight into LDS (buffer loads with the LDS bit), row by row for merged loads: LDS slot
+  // q = m * L + sq holds piece sq ^ (m % 16) of row m, rows m >= M read as zero (6 x 5120 -> 1024 7.1 ->
+  // 6.5 us against A-fragment order). A wave's instruction fills 64 consecutive slots
+  // (the instruction's base + 16 lane); the slot count L * MP is a multiple of 64, so a wave
   // either fills whole slots or skips the instruction.
   typedef __attribute__((address_space(3))) void* lds_ptr;
   auto dma_x_all = [&]() __attribute__((always_inline)) {
-    const int slots = S * 16 * MP;
+    const int slots = L * MP;
 #pragma unroll
     for (int j = 0; j < kRsSmallXP; ++j) {
       const int base = j * kRsThreads + 64 * wave;
       if (base < slots) {
         const int q = base + lane;
-        const int sq = q / MP, m = q - sq * MP;
+        const int m = q / L, sq = (q - m * L) ^ (m & 15);
         const uint32_t off = m < P.M ? ((uint32_t)m * (uint32_t)P.K + (uint32_t)sq * 8u) * 2u : 0x80000000u;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(lds + (size_t)base * 16), 16, off, 0, 0, 0);
       }
@@ -357,7 +398,7 @@ void rowsplit_kernel(RowSplitParams P) {
         if (grp < P.M && c < (P.K >> 3)) {
           const u32x4 nv = norm_scale_chunk(nx[q][i], nwt[i], inv);
           const int sq = c - (kq >> 3);
-          if (sq >= 0 && sq < S * 16) xs[sq * MP + grp] = nv;
+          if (sq >= 0 && sq < L) xs[sq * MP + grp] = nv;
           if (first) {
             const size_t o = (size_t)grp * P.K + (size_t)c * 8;
             *reinterpret_cast<u32x4*>(P.h_out + o) = nx[q][i];
@@ -385,13 +426,15 @@ void rowsplit_kernel(RowSplitParams P) {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  const int aoff = g * 4 * MP + min(n, P.M - 1);
+  // Fragment reads: lane (n, g) reads piece 16 v + 4 g + tt of row min(n, M - 1).
+  const int arow = min(n, P.M - 1);
+  const int aoff = ROWX ? arow * L : g * 4 * MP + (MERGE ? arow ^ g : arow);
   int ndone = 0;
   __builtin_amdgcn_s_setprio(3);
 
   auto compute = [&](int j, int st, auto fast, f32x4 acc) __attribute__((always_inline)) {
     constexpr bool FAST = decltype(fast)::value;
-    const u32x4* xb = xs + (size_t)st * V * 16 * MP;
+    const u32x4* xb = xs + (size_t)st * V * 16 * (ROWX ? 1 : MP);
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       const int e2 = 2 * v + (g >> 1);
@@ -403,11 +446,22 @@ void rowsplit_kernel(RowSplitParams P) {
 #pragma unroll
       for (int tt = 0; tt < 4; ++tt) {
         const u32x4 B = FAST ? dequant_word_fast(wv[j][v][tt], c1, c2, bf) : dequant_word(wv[j][v][tt], c1, c2, bf);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xb[(v * 16 + tt) * MP + aoff]), as_bf16x8(B), acc,
-                                                      0, 0, 0);
+        const u32x4 A = xb[ROWX ? aoff + v * 16 + ((4 * g + tt) ^ arow) : (v * 16 + tt) * MP + aoff];
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(A), as_bf16x8(B), acc, 0, 0, 0);
       }
     }
     return acc;
+  };
+  // Ring slot j's unit (step st of its block) added to acc.
+  auto unit_sum = [&](int j, int st, f32x4 acc) __attribute__((always_inline)) {
+    bool bad = false;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const int e2 = 2 * v + (g >> 1);
+      bad |= !fast_scale_ok((sv[j].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
+    }
+    if (__builtin_amdgcn_ballot_w64(bad) == 0) return compute(j, st, std::true_type{}, acc);
+    return compute(j, st, std::false_type{}, acc);
   };
 
   // One unit from ring slot J: take the next unit index (its LDS round trip overlaps the MFMAs),
@@ -418,18 +472,7 @@ void rowsplit_kernel(RowSplitParams P) {
     if (lane == 0) taken = __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     const int nu = __builtin_amdgcn_readfirstlane(taken);
     const int b = u / SU, st = u - b * SU;
-    bool bad = false;
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const int e2 = 2 * v + (g >> 1);
-      bad |= !fast_scale_ok((sv[j].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-    }
-    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    f32x4 acc;
-    if (__builtin_amdgcn_ballot_w64(bad) == 0)
-      acc = compute(j, st, std::true_type{}, zero);
-    else
-      acc = compute(j, st, std::false_type{}, zero);
+    const f32x4 acc = unit_sum(j, st, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
     if (g < G) part[(u * G + g) * 16 + n] = acc;
     ++ndone;
     // A wave's issue priority falls with the units it has done: the SIMD arbiter otherwise
@@ -444,22 +487,9 @@ void rowsplit_kernel(RowSplitParams P) {
 
   if constexpr (SMALL) {
     // Units w and w + 16 (both in the ring since the start), sums kept until x is dead.
-    auto unit_sums = [&](int u, auto jc) __attribute__((always_inline)) {
-      constexpr int j = decltype(jc)::value;
-      const int st = u - (u / SU) * SU;
-      bool bad = false;
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const int e2 = 2 * v + (g >> 1);
-        bad |= !fast_scale_ok((sv[j].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-      }
-      const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (__builtin_amdgcn_ballot_w64(bad) == 0) return compute(j, st, std::true_type{}, zero);
-      return compute(j, st, std::false_type{}, zero);
-    };
     f32x4 acc0 = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = acc0;
-    if (ua < U) acc0 = unit_sums(ua, std::integral_constant<int, 0>{});
-    if (ub < U) acc1 = unit_sums(ub, std::integral_constant<int, 1>{});
+    if (ua < U) acc0 = unit_sum(0, ua - (ua / SU) * SU, acc0);
+    if (ub < U) acc1 = unit_sum(1, ub - (ub / SU) * SU, acc1);
     __syncthreads();
     if (g < G) {
       if (ua < U) part[(ua * G + g) * 16 + n] = acc0;
@@ -475,16 +505,7 @@ void rowsplit_kernel(RowSplitParams P) {
     auto step = [&](int q, int& u, auto jc) __attribute__((always_inline)) {
       constexpr int j = decltype(jc)::value;
       const int b = u / SU, st = u - b * SU;
-      bool bad = false;
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const int e2 = 2 * v + (g >> 1);
-        bad |= !fast_scale_ok((sv[j].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-      }
-      if (__builtin_amdgcn_ballot_w64(bad) == 0)
-        acc = compute(j, st, std::true_type{}, acc);
-      else
-        acc = compute(j, st, std::false_type{}, acc);
+      acc = unit_sum(j, st, acc);
       u = own_unit(q + 2);
       fetch(j, u);
       if (st == SU - 1) {
@@ -517,18 +538,6 @@ void rowsplit_kernel(RowSplitParams P) {
     // into the group's sums, the slot is refilled with the unit two ahead; a group's sums go to
     // its slot after its last unit.
     const int GU = P.GU;
-    auto one = [&](int u, auto jc, f32x4 acc) __attribute__((always_inline)) {
-      constexpr int j = decltype(jc)::value;
-      const int st = u - (u / SU) * SU;
-      bool bad = false;
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const int e2 = 2 * v + (g >> 1);
-        bad |= !fast_scale_ok((sv[j].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-      }
-      if (__builtin_amdgcn_ballot_w64(bad) == 0) return compute(j, st, std::true_type{}, acc);
-      return compute(j, st, std::false_type{}, acc);
-    };
     // (A group taken one group ahead, to hide the atomic's round trip, made pairs 9% slower.)
     auto succ = [&](int u) __attribute__((always_inline)) {
       if ((u + 1) % GU != 0) return u + 1;
@@ -540,7 +549,7 @@ void rowsplit_kernel(RowSplitParams P) {
     // Slot J's unit u is computed, then u becomes the unit after `other` (the next in sequence).
     auto step = [&](int& u, int other, auto jc) __attribute__((always_inline)) {
       constexpr int j = decltype(jc)::value;
-      acc = one(u, jc, acc);
+      acc = unit_sum(j, u - (u / SU) * SU, acc);
       if ((u + 1) % GU == 0) {
         if (g < G) part[((u / GU) * G + g) * 16 + n] = acc;
         acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -559,9 +568,9 @@ void rowsplit_kernel(RowSplitParams P) {
         int taken = 0;
         if (lane == 0) taken = __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         const int np = __builtin_amdgcn_readfirstlane(taken);
-        acc = one(ua, std::integral_constant<int, 0>{}, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+        acc = unit_sum(0, ua - (ua / SU) * SU, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
         fetch(0, 2 * np);
-        acc = one(ub, std::integral_constant<int, 1>{}, acc);
+        acc = unit_sum(1, ub - (ub / SU) * SU, acc);
         if (g < G) part[((ua >> 1) * G + g) * 16 + n] = acc;
         ++ndone;
         if (ndone == 1) __builtin_amdgcn_s_setprio(2);
@@ -671,126 +680,141 @@ void rowsplit_kernel(RowSplitParams P) {
   if (tid == 0) __hip_atomic_store(&P.cnt[range], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Up to 16 rows of x over a small problem, whole K per workgroup, x never staged: workgroup p owns
-// the R <= 32 rows [p R, p R + R) (RB <= 2 blocks of 16) and has one wave per K chunk of 512 k
-// (at most 12: K <= 6144, three waves per SIMD, 170 registers each). Wave w computes chunk w for
-// every block: it loads the chunk's A fragments of x (16 rows x 512 k,
-// lane (m, g) holds x[min(m, M - 1)] at the MFMA's k) straight into registers, the chunk's weights,
-// scales and biases of both blocks, and runs the chunk's MFMAs with each A fragment feeding both
-// blocks. Every load of the workgroup is issued at the start and nothing waits for a barrier
-// before the first MFMA; the chunk sums meet in LDS (one slot per chunk and block) and are added
-// in chunk order (deterministic). One memory round trip plus the L2 reads of x bound such a
-// launch (a verify tile of 16 x 5120 over 5120 columns: 160 KB of x per CU from L2, 57 KB of
-// weights from HBM).
+// Up to 16 rows of x over a small problem, whole K per workgroup: workgroup p owns the R <= 32 rows
+// [p R, p R + R) (RB <= 2 blocks of 16) and has one wave per K chunk of 512 k (at most 12: K <= 6144,
+// three waves per SIMD). Wave w computes chunk w for every block: it loads the chunk's x (16 rows x
+// 512 k), weights, scales and biases into registers, all at the start, x and the scales with four or
+// more neighbouring lanes per row (merged by the address unit), and puts x, half a chunk at a time,
+// and the scales in MFMA order through LDS of its own: no barrier before the chunk sums, which meet
+// in LDS (one slot per chunk and block) and are added in chunk order (deterministic). One memory
+// round trip plus the L2 reads of x bound such a launch (a verify tile of 16 x 5120 over 5120
+// columns: 160 KB of x per CU from L2, 57 KB of weights from HBM). Loading x straight in MFMA order
+// (one row per neighbouring lane, 37 against 86 GB/s per CU) took 16 / 9 x 5120 -> 5120 11.7 / 10.5 us
+// against 8.9 / 8.8, 10 x 4096 -> 4096 7.7 against 6.7; a streaming read of the weights alone 3.9.
 constexpr int kXrV = 4;        // super-steps per chunk (512 k)
 constexpr int kXrMaxRB = 2;    // blocks per workgroup
 constexpr int kXrMaxWaves = 12;
-template <int NCH>
+constexpr size_t kXrHalf = 16 * 512;            // LDS bytes of half a chunk of x (16 rows x 256 k)
+static_assert(kXrMaxWaves * ((size_t)kXrMaxRB * 4 * 16 * 16 + kXrHalf + (size_t)kXrMaxRB * 2 * 16 * 16) <= kRsLds, "LDS");
+constexpr size_t kXrSc = kXrMaxRB * 2 * 16 * 16;  // LDS bytes of a chunk's scales and biases
+// Dynamic LDS: [chunk][block][4 groups][16 lanes] f32x4 sums, then per wave its half chunk of x and
+// its scales and biases.
+__host__ __device__ inline size_t xreg_part_bytes(int SU) { return (size_t)SU * kXrMaxRB * 4 * 16 * 16; }
 __global__ __launch_bounds__(64 * kXrMaxWaves) __attribute__((amdgpu_waves_per_eu(3)))
 void rowsplit_xreg_kernel(RowSplitParams P) {
   constexpr int V = kXrV;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  f32x4* part = reinterpret_cast<f32x4*>(lds);  // [chunk][block][4 groups][16 lanes]
+  f32x4* part = reinterpret_cast<f32x4*>(lds);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
-  const int SU = P.SU;  // chunks along K
+  const int SU = P.SU;  // chunks along K, one per wave
   const int RB = P.RB;
   const int r0 = blockIdx.x * P.R;
   const int r1 = min(P.N, r0 + P.R);
   const int KG = P.K >> 6;
+  const int st = wave;
   constexpr uint32_t kOut = 0x40000000u;  // past the end of every buffer (each below 1 GiB)
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(P.x), 0, rsrc_bytes((unsigned long long)P.M * P.K * 2), kBufferRsrcWord3);
-  const int wrec = rsrc_bytes((unsigned long long)P.N * (P.K >> 1));
-  const int srec = rsrc_bytes((unsigned long long)P.N * KG * 2);
-  const uint32_t xrow = (uint32_t)min(n, P.M - 1) * (uint32_t)P.K * 2u;
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint32_t*>(P.w), 0, rsrc_bytes((unsigned long long)P.N * (P.K >> 1)), kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(P.s), 0, rsrc_bytes((unsigned long long)P.N * KG * 2), kBufferRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(P.b), 0, rsrc_bytes((unsigned long long)P.N * KG * 2), kBufferRsrcWord3);
+  uint8_t* const xw = lds + xreg_part_bytes(SU) + (size_t)wave * (kXrHalf + kXrSc);
+  uint8_t* const scw = xw + kXrHalf;
 
-  u32x4 xa[NCH][V][4];
-  u32x4 wv[NCH][kXrMaxRB][V];
-  Scales<V> sv[NCH][kXrMaxRB], bv[NCH][kXrMaxRB];
-  // Issue every load of this wave's chunks in two halves of its super-steps, each half's weights
+  u32x4 xa[2][8];  // half h of the chunk's x: row 2 i + lane / 32, 16-byte piece lane % 32 of its 512 bytes
+  u32x4 wv[kXrMaxRB][V];
+  uint32_t sv[kXrMaxRB], bv[kXrMaxRB];  // dword lane % 4 of row lane / 4's 8 scales (biases)
+  // Issue every load of this wave's chunk in two halves of its super-steps, each half's weights
   // (from HBM) before its x (from L2): the first half's MFMAs need only the first half's loads
   // (16 x 5120 -> 5120 14.5 -> 14.3 us, 9 rows 13.1 -> 12.9 us; quarters were no better).
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int st = wave + c * kXrMaxWaves;
-      const bool live = st < SU;
-      const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(P.w), 0,
-                                                                          live ? wrec : 0, kBufferRsrcWord3);
-      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(P.s), 0,
-                                                                          live ? srec : 0, kBufferRsrcWord3);
-      const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(P.b), 0,
-                                                                          live ? srec : 0, kBufferRsrcWord3);
-#pragma unroll
-      for (int b = 0; b < kXrMaxRB; ++b) {
-        const int row = r0 + b * 16 + n;
-        const bool ok = b < RB && row < r1;
-        const uint32_t wo = ok ? (uint32_t)row * (uint32_t)(P.K >> 1) + (uint32_t)g * 16u : kOut;
-        const uint32_t so = ok ? (uint32_t)row * (uint32_t)KG * 2u : kOut;
-        if (h == 0) {
-          sv[c][b] = load_scales<V>(rs, so, live ? st * 4 * V : 0);
-          bv[c][b] = load_scales<V>(rb, so, live ? st * 4 * V : 0);
-        }
-#pragma unroll
-        for (int v = h * V / 2; v < (h + 1) * V / 2; ++v)
-          wv[c][b][v] = __builtin_amdgcn_raw_buffer_load_b128(rw, wo + v * 64, live ? st * V * 64 : 0, 0);
+    for (int b = 0; b < kXrMaxRB; ++b) {
+      const int row = r0 + b * 16 + n, row4 = r0 + b * 16 + (lane >> 2);
+      const uint32_t wo = b < RB && row < r1 ? (uint32_t)row * (uint32_t)(P.K >> 1) + (uint32_t)g * 16u : kOut;
+      if (h == 0) {
+        const uint32_t so = b < RB && row4 < r1 ? (uint32_t)row4 * (uint32_t)KG * 2u + (uint32_t)(lane & 3) * 4u : kOut;
+        sv[b] = __builtin_amdgcn_raw_buffer_load_b32(rs, so, st * 4 * V, 0);
+        bv[b] = __builtin_amdgcn_raw_buffer_load_b32(rb, so, st * 4 * V, 0);
       }
 #pragma unroll
       for (int v = h * V / 2; v < (h + 1) * V / 2; ++v)
+        wv[b][v] = __builtin_amdgcn_raw_buffer_load_b128(rw, wo + v * 64, st * V * 64, 0);
+    }
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
-          const uint32_t off = live ? xrow + (uint32_t)(st * V * 128 + v * 128 + g * 32 + tt * 8) * 2u : 0x80000000u;
-          xa[c][v][tt] = __builtin_amdgcn_raw_buffer_load_b128(rx, off, 0, 0);
-        }
+    for (int i = 0; i < 8; ++i) {
+      const int m = 2 * i + (lane >> 5);
+      const uint32_t off = m < P.M ? (uint32_t)m * (uint32_t)P.K * 2u + (uint32_t)(lane & 31) * 16u : 0x80000000u;
+      xa[h][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, off, (st * V * 128 + h * 256) * 2, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   }
 
+  // Everything below, up to the chunk sums, stays within the wave (its own LDS, accessed in order).
+  bool bad = false;
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    const int st = wave + c * kXrMaxWaves;
-    if (st >= SU) break;
-    f32x4 acc[kXrMaxRB];
+  for (int b = 0; b < kXrMaxRB; ++b) {
+    reinterpret_cast<uint32_t*>(scw)[b * 128 + lane] = sv[b];
+    reinterpret_cast<uint32_t*>(scw)[b * 128 + 64 + lane] = bv[b];
+    bad |= !fast_scale_ok(sv[b] & 0xFFFFu) || !fast_scale_ok(sv[b] >> 16);
+  }
+  const bool fast = __builtin_amdgcn_ballot_w64(bad) == 0;
+  f32x4 acc[kXrMaxRB];
 #pragma unroll
-    for (int b = 0; b < kXrMaxRB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    bool bad = false;
+  for (int b = 0; b < kXrMaxRB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  u32x4* const xl = reinterpret_cast<u32x4*>(xw);
+  const uint16_t* const ssl = reinterpret_cast<const uint16_t*>(scw + n * 16) + (g >> 1);
+  auto half = [&](auto hc, auto fc) __attribute__((always_inline)) {
+    constexpr int h = decltype(hc)::value;
+    constexpr bool FAST = decltype(fc)::value;
 #pragma unroll
-    for (int b = 0; b < kXrMaxRB; ++b)
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const int e2 = 2 * v + (g >> 1);
-        bad |= !fast_scale_ok((sv[c][b].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-      }
-    const bool fast = __builtin_amdgcn_ballot_w64(bad) == 0;
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-      const int e2 = 2 * v + (g >> 1);
+    for (int v = h * V / 2; v < (h + 1) * V / 2; ++v) {
       float c1[kXrMaxRB], c2[kXrMaxRB], bf[kXrMaxRB];
 #pragma unroll
       for (int b = 0; b < kXrMaxRB; ++b) {
-        const float sf = bf16_to_f32((sv[c][b].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-        bf[b] = bf16_to_f32((bv[c][b].d[e2 >> 1] >> (16 * (e2 & 1))) & 0xFFFFu);
-        c1[b] = fast ? sf * 16777216.0f : sf;
-        c2[b] = fast ? sf * 1048576.0f : sf * 0.0625f;
+        const float sf = bf16_to_f32(ssl[b * 256 + 2 * v]);
+        bf[b] = bf16_to_f32(ssl[b * 256 + 128 + 2 * v]);
+        c1[b] = FAST ? sf * 16777216.0f : sf;
+        c2[b] = FAST ? sf * 1048576.0f : sf * 0.0625f;
       }
 #pragma unroll
-      for (int tt = 0; tt < 4; ++tt)
+      for (int tt = 0; tt < 4; ++tt) {
+        const u32x4 A = xl[n * 32 + (v & 1) * 16 + ((4 * g + tt) ^ n)];
 #pragma unroll
         for (int b = 0; b < kXrMaxRB; ++b) {
           if (b < RB) {
-            const u32x4 B = fast ? dequant_word_fast(wv[c][b][v][tt], c1[b], c2[b], bf[b])
-                                 : dequant_word(wv[c][b][v][tt], c1[b], c2[b], bf[b]);
-            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xa[c][v][tt]), as_bf16x8(B), acc[b], 0, 0, 0);
+            const u32x4 B = FAST ? dequant_word_fast(wv[b][v][tt], c1[b], c2[b], bf[b])
+                                 : dequant_word(wv[b][v][tt], c1[b], c2[b], bf[b]);
+            acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(A), as_bf16x8(B), acc[b], 0, 0, 0);
           }
         }
+      }
     }
+  };
+  auto put_x = [&](int h) __attribute__((always_inline)) {
+    wave_lds_order();
 #pragma unroll
-    for (int b = 0; b < kXrMaxRB; ++b)
-      if (b < RB) part[((st * kXrMaxRB + b) * 4 + g) * 16 + n] = acc[b];
-  }
+    for (int i = 0; i < 8; ++i) {
+      const int m = 2 * i + (lane >> 5);
+      xl[m * 32 + ((lane & 31) ^ m)] = xa[h][i];
+    }
+    wave_lds_order();
+  };
+  put_x(0);
+  if (fast) half(std::integral_constant<int, 0>{}, std::true_type{});
+  else half(std::integral_constant<int, 0>{}, std::false_type{});
+  put_x(1);
+  if (fast) half(std::integral_constant<int, 1>{}, std::true_type{});
+  else half(std::integral_constant<int, 1>{}, std::false_type{});
+#pragma unroll
+  for (int b = 0; b < kXrMaxRB; ++b)
+    if (b < RB) part[((st * kXrMaxRB + b) * 4 + g) * 16 + n] = acc[b];
   __syncthreads();
 
   // y[m, col]: the chunk sums of the column's block in chunk order; output row m = 4 g + r.
@@ -841,7 +865,7 @@ bool rowsplit_xreg_plan(int M, int N, int K, int cus, RowSplitPlan* plan) {
   plan->ranges = (N + R - 1) / R;
   plan->blocks = plan->ranges;
   plan->part_bytes = 0;
-  plan->smem = (size_t)SU * kXrMaxRB * 4 * 16 * 16;
+  plan->smem = xreg_part_bytes(SU);  // the chunk sums; the launch adds each wave's own LDS
   return true;
 }
 
@@ -1023,7 +1047,15 @@ hipError_t launch_rowsplit_m(const RowSplitPlan& plan, const RowSplitParams& P, 
 }
 
 hipError_t launch_rowsplit_xreg(const RowSplitPlan& plan, const RowSplitParams& P, hipStream_t stream) {
-  hipLaunchKernelGGL((rowsplit_xreg_kernel<1>), dim3(plan.blocks), dim3(64 * plan.SU), plan.smem, stream, P);
+  static bool attr_set = false;  // the attribute is per function; setting it twice is harmless
+  if (!attr_set) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&rowsplit_xreg_kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRsLds);
+    if (e != hipSuccess) return e;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(rowsplit_xreg_kernel, dim3(plan.blocks), dim3(64 * plan.SU),
+                     plan.smem + (size_t)plan.SU * (kXrHalf + kXrSc), stream, P);
   return hipGetLastError();
 }
 
