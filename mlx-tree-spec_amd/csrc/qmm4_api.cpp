@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "qmm4.h"
+#include "qmm_general.h"
 #include "qmm4_dispatch.h"
 #include "qmm4_kernels.h"
 
@@ -631,6 +632,46 @@ int qmm4_add_rms_norm_bf16(const void* x, const void* r, const void* weight, voi
                                            static_cast<uint16_t*>(n_out), (int)rows, (int)D, eps,
                                            static_cast<hipStream_t>(hip_stream));
   if (e != hipSuccess) return hip_error(e, "add-rms-norm kernel launch");
+  return QMM4_OK;
+}
+
+int qmm_affine_general_bf16(const void* x, const uint32_t* w, const void* scales, const void* biases, void* y,
+                            int64_t M, int64_t N, int64_t K, int group_size, int bits, void* hip_stream) {
+  qmm4::clear_error();
+  if (bits != 2 && bits != 4 && bits != 8)
+    return set_error(QMM4_ERR_UNSUPPORTED, "bits=%d: 2-, 4- and 8-bit codes are supported", bits);
+  if (group_size != 32 && group_size != 64 && group_size != 128)
+    return set_error(QMM4_ERR_UNSUPPORTED, "group_size=%d: groups of 32, 64 and 128 are supported", group_size);
+  if (M < 0 || N < 0 || K <= 0 || K % 64 != 0 || K % group_size != 0)
+    return set_error(QMM4_ERR_INVALID, "invalid shape M=%lld N=%lld K=%lld (K must be a positive multiple of 64 and of "
+                     "group_size=%d)", (long long)M, (long long)N, (long long)K, group_size);
+  if (M > (1LL << 20) || N > (1LL << 30) || K > (1LL << 24))
+    return set_error(QMM4_ERR_INVALID, "shape M=%lld N=%lld K=%lld is too large", (long long)M, (long long)N, (long long)K);
+  if (M == 0 || N == 0) return QMM4_OK;
+  if (!x || !w || !scales || !biases || !y) return set_error(QMM4_ERR_INVALID, "null pointer argument");
+  if (!aligned(x, 16) || !aligned(w, 16)) return set_error(QMM4_ERR_INVALID, "x and w must be 16-byte aligned");
+  if (!aligned(scales, 2) || !aligned(biases, 2) || !aligned(y, 2))
+    return set_error(QMM4_ERR_INVALID, "scales, biases and y must be 2-byte aligned");
+  // Byte offsets (which may reach 64 rows or columns past the end) stay below 2 GiB.
+  constexpr unsigned long long kMax = 1ULL << 31;
+  if ((unsigned long long)(M + 64) * K * 2 >= kMax || (unsigned long long)(N + 64) * (K / 8 * bits) >= kMax ||
+      (unsigned long long)(N + 64) * (K / 32) * 2 >= kMax)
+    return set_error(QMM4_ERR_INVALID, "x [%lld, %lld] or w [%lld, %lld] exceeds 2 GiB", (long long)M, (long long)K,
+                     (long long)N, (long long)K);
+  int dev = 0;
+  int rc = current_device(&dev);
+  if (rc) return rc;
+  int cus = 0;
+  {
+    std::lock_guard<std::mutex> lock(qmm4::api_mutex());
+    qmm4::DeviceInfo* di = nullptr;
+    if ((rc = qmm4::device_info(dev, &di))) return rc;
+    cus = qmm4::device_cus(di);
+  }
+  hipError_t e = qmm4::launch_general(static_cast<const uint16_t*>(x), w, static_cast<const uint16_t*>(scales),
+                                      static_cast<const uint16_t*>(biases), static_cast<uint16_t*>(y), (int)M, (int)N,
+                                      (int)K, group_size, bits, cus, static_cast<hipStream_t>(hip_stream));
+  if (e != hipSuccess) return hip_error(e, "general quantized matmul kernel launch");
   return QMM4_OK;
 }
 

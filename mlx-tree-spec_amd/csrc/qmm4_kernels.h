@@ -158,4 +158,9 @@ hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* 
 hipError_t launch_dequant(const uint32_t* w, const uint16_t* s, const uint16_t* b, uint16_t* out, int64_t N,
                           int64_t K, int group_size, int bits, hipStream_t stream);
 
+// y = x @ dequant(w)^T in the formats and shapes the packed kernels do not take: 2-, 4- or 8-bit codes
+// in groups of 32, 64 or 128, any N, K % 64 == 0; x, w, the scales and the biases each below 2 GiB.
+hipError_t launch_general(const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b, uint16_t* y,
+                          int M, int N, int K, int group_size, int bits, int cus, hipStream_t stream);
+
 }  // namespace qmm4

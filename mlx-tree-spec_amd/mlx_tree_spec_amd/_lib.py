@@ -24,7 +24,7 @@ QMM4_EPILOGUE_SILU_MUL = 1
 # Size of qmm4_affine_bf16_noalloc's static device array per GPU (QMM4_NOALLOC_SCRATCH_BYTES).
 QMM4_NOALLOC_SCRATCH_BYTES = 136 * 1024 * 1024
 
-# name -> (restype, argtypes); the symbols include/qmm4.h declares.
+# name -> (restype, argtypes); the symbols include/qmm4.h and include/qmm_general.h declare.
 _vp = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _int = ctypes.c_int
@@ -36,6 +36,7 @@ SIGNATURES = {
     "qmm4_add_rms_norm_bf16": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, ctypes.c_float, _vp]),
     "qmm4_add_rms_norm_qmm_bf16": (_int, [_vp, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _i64, _i64, _i64, _int, _int, _int, _int, _vp]),
+    "qmm_affine_general_bf16": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _int, _vp]),
     "qmm4_last_error": (ctypes.c_char_p, []),
     "qmm4_abi_version": (_int, []),
 }

@@ -26,8 +26,8 @@ _W_DTYPES = (torch.int32, torch.uint32)
 
 # MLX affine formats whose codes fill whole uint32 words (code k = (32 / bits) c + i in bits
 # [bits i, bits i + bits) of word c): dequantize takes them all, and so does quantized_matmul,
-# whose packed kernels implement 4 bits in groups of 64 (other formats: dequantize, then a bf16
-# GEMM, as the reference leaves them to MLX's own op, packed_linear.py:84-86). 3-, 5- and 6-bit
+# whose packed kernels implement 4 bits in groups of 64 (other formats: the general kernel, or
+# dequantize and a bf16 GEMM; the reference leaves them to MLX's own op, packed_linear.py:84-86). 3-, 5- and 6-bit
 # codes, which MLX packs across word boundaries, are not supported.
 GENERAL_BITS = (2, 4, 8)
 GENERAL_GROUP_SIZES = (32, 64, 128)
@@ -92,6 +92,26 @@ def aligned_contiguous(t: torch.Tensor, align: int = 16) -> torch.Tensor:
 
 
 
+# The general kernel dequantizes the weights once per 64 rows, the other form once and runs a library
+# product: 256 x 8192 -> 8191 90 against 137 us, 512 rows 160 against 118; small products stay with the
+# kernel past 256 rows (512 x 1024 -> 513 6.7 against 29 us, 512 x 2560 -> 4101 41 against 34).
+GENERAL_KERNEL_MAX_ROWS = 256
+GENERAL_KERNEL_MAX_PRODUCT = 1 << 31
+
+
+def _general_kernel_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bool:
+    """Whether the general kernel takes this product: K a multiple of its 64-k unit, up to 256 rows or a
+    small product, byte offsets (with up to 64 rows past the end) below 2 GiB, and no gradient asked
+    of x (the library product is differentiable in x; the kernels are not)."""
+    if k % 64 or m == 0 or n == 0 or not (m <= GENERAL_KERNEL_MAX_ROWS or m * n * k <= GENERAL_KERNEL_MAX_PRODUCT):
+        return False
+    if (m + 64) * k * 2 >= 1 << 31 or (n + 64) * (k // 8 * bits) >= 1 << 31 or (n + 64) * (k // 32) * 2 >= 1 << 31:
+        return False
+    if m > 1 << 20 or n > 1 << 30 or k > 1 << 24:
+        return False
+    return not (x.requires_grad and torch.is_grad_enabled()) and torch.autograd.forward_ad._current_level < 0
+
+
 def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                      transpose: bool = True, group_size: int = 64, bits: int = 4,
                      mode: str = "affine") -> torch.Tensor:
@@ -99,8 +119,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
 
     Shapes the packed kernels take (4-bit codes in groups of 64, K % 128 == 0, N % 16 == 0) run
     them. Other shapes (K % 64 == 0, any N) and formats (2-, 4- or 8-bit codes in groups of 32, 64
-    or 128) are what the reference leaves to MLX's own op (packed_linear.py:56-57, 84-86): the
-    weights are dequantized exactly by the HIP kernel and multiplied by a bf16 GEMM with fp32
+    or 128) are what the reference leaves to MLX's own op (packed_linear.py:56-57, 84-86): up to 256
+    rows (more over small weights; K % 64 == 0) run the general kernel, which dequantizes exactly in
+    registers; others dequantize the weights and multiply by a bf16 GEMM, both with fp32
     accumulation on the same stream.
     """
     _check_format(group_size, bits, transpose, mode, general=True)
@@ -116,6 +137,18 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     x2 = aligned_contiguous(x.reshape(-1, k))
     m = x2.shape[0]
     if k % 128 or n % 16 or bits != 4 or group_size != 64:
+        if _general_kernel_ok(x, m, n, k, bits):
+            w = aligned_contiguous(w)
+            scales = aligned_contiguous(scales, 2)
+            biases = aligned_contiguous(biases, 2)
+            y = torch.empty((*x.shape[:-1], n), dtype=torch.bfloat16, device=dev)
+            lib = _lib.load()
+            with torch.cuda.device(dev):
+                stream = torch.cuda.current_stream(dev).cuda_stream
+                rc = lib.qmm_affine_general_bf16(x2.data_ptr(), w.data_ptr(), scales.data_ptr(), biases.data_ptr(),
+                                                 y.data_ptr(), m, n, k, group_size, bits, stream)
+            _lib.check(rc, "quantized_matmul")
+            return y
         wd = dequantize(w, scales, biases, group_size, bits)
         return torch.nn.functional.linear(x2, wd).reshape(*x.shape[:-1], n)
     w = aligned_contiguous(w)
