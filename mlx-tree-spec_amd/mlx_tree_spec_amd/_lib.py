@@ -66,6 +66,30 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The native form of the package's calls (csrc/host/native.cpp), bound to the loaded library.
+
+    Its functions take the usual call (plain contiguous aligned tensors on the current device) and
+    return None for anything else, or a negative error code of the library."""
+    global _native
+    if _native is None:
+        lib = load()
+        if not os.path.exists(os.path.join(_HERE, "_native.so")):
+            raise LibraryNotBuilt(f"{_HERE}/_native.so not found: build it with `python -m mlx_tree_spec_amd.build` "
+                                  "(or __graft_entry__.build())")
+        import torch  # noqa: F401  (its libraries are what the extension links to)
+
+        from . import _native as mod
+        mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+            "qmm4_affine_bf16", "qmm4_gate_up_silu_bf16", "qmm_affine_general_bf16", "qmm4_add_rms_norm_bf16",
+            "qmm4_add_rms_norm_qmm_bf16")))
+        _native = mod
+    return _native
+
+
 def last_error() -> str:
     msg = load().qmm4_last_error()
     return msg.decode() if msg else ""

@@ -2,6 +2,9 @@
 
     python -m mlx_tree_spec_amd.build      (with mlx-tree-spec_amd/ on sys.path)
 
+_native.so (csrc/host/, the calls of the package from tensors to the C ABI) is a CPython extension on
+libtorch, built with the host compiler.
+
 Objects compile in parallel; the library is linked to a temporary name and renamed, so a reader
 never sees a half-written file.
 """
@@ -12,6 +15,7 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -25,6 +29,8 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 # of its own that only bench.py loads.
 FLOOR_DIR = os.path.join(CSRC, "floor")
 FLOOR_PATH = os.path.join(PKG_DIR, "libqmm4_floor.so")
+HOST_DIR = os.path.join(CSRC, "host")
+NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
 ARCH = os.environ.get("QMM4_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops off: no v_pk_{add,mul,fma}_f32 in device code. hipcc's host pass warns that
@@ -61,11 +67,33 @@ def _link(srcs: list[str], out: str) -> None:
         os.replace(out_tmp, out)
 
 
+def _build_native(out: str) -> None:
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    lib = os.path.join(root, "lib")
+    out_tmp = out + f".tmp{os.getpid()}"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
+           "-I", sysconfig.get_paths()["include"], "-I", os.path.join(root, "include"),
+           "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-I", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+           *sorted(os.path.join(HOST_DIR, f) for f in os.listdir(HOST_DIR) if f.endswith(".cpp")),
+           "-L", lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-o", out_tmp]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"building {out} failed:\n{r.stdout}\n{r.stderr}")
+    os.replace(out_tmp, out)
+
+
 def build(verbose: bool = False) -> str:
-    _link(sources(), LIB_PATH)
+    with cf.ThreadPoolExecutor(max_workers=1) as ex:
+        native = ex.submit(_build_native, NATIVE_PATH)
+        _link(sources(), LIB_PATH)
+        native.result()
     _link(sorted(os.path.join(FLOOR_DIR, f) for f in os.listdir(FLOOR_DIR) if f.endswith(".hip")), FLOOR_PATH)
     if verbose:
-        print(f"built {LIB_PATH} and {FLOOR_PATH}")
+        print(f"built {LIB_PATH}, {NATIVE_PATH} and {FLOOR_PATH}")
     return LIB_PATH
 
 

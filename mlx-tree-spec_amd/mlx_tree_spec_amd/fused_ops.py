@@ -24,6 +24,12 @@ from .qmm import _check_device, _check_format, _check_weights, aligned_contiguou
 def add_rms_norm_(x: torch.Tensor, r: torch.Tensor, weight: torch.Tensor, eps: float):
     """(x + r, rmsnorm(x + r) * weight) as bf16, each shaped like x: h = bf16(x + r),
     n = bf16(weight * bf16(h / sqrt(mean(h^2) + eps))) over the last dimension."""
+    if x.is_cuda:
+        out = _lib.native().norm(x, r, weight, float(eps))
+        if type(out) is int:
+            _lib.check(out, "add_rms_norm")
+        if out is not None:
+            return out
     for name, t in (("x", x), ("r", r), ("weight", weight)):
         if t.dtype != torch.bfloat16:
             raise ValueError(f"[add_rms_norm] {name} must be bfloat16, got {t.dtype}")
@@ -60,8 +66,14 @@ def add_rms_norm_qmm_(x: torch.Tensor, r: torch.Tensor, weight: torch.Tensor, ep
     """(h, n, y): h, n = add_rms_norm_(x, r, weight, eps) and y = quantized_matmul(n, w, scales,
     biases) (or gate_up_silu(n, w, scales, biases) when silu_mul), bit for bit, in one launch when
     the projection runs as the row-split kernel (up to 4 rows, K <= 8192)."""
-    _check_format(group_size, bits)
     what = "add_rms_norm_qmm"
+    if bits == 4 and group_size == 64 and x.is_cuda:
+        out = _lib.native().norm_qmm(x, r, weight, float(eps), w, scales, biases, bool(silu_mul))
+        if type(out) is int:
+            _lib.check(out, what)
+        if out is not None:
+            return out
+    _check_format(group_size, bits)
     for name, t in (("x", x), ("r", r), ("weight", weight)):
         if t.dtype != torch.bfloat16:
             raise ValueError(f"[{what}] {name} must be bfloat16, got {t.dtype}")

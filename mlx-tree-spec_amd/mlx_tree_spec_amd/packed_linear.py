@@ -153,8 +153,17 @@ def _launcher(mod: QuantizedLinear):
     wp, sp, bp = w.data_ptr(), s.data_ptr(), b.data_ptr()
     dev = w.device
     fn = _lib.load().qmm4_affine_bf16
+    linear = _lib.native().linear
 
     def run(x: torch.Tensor) -> torch.Tensor | None:
+        bufs = mod._buffers
+        if bufs.get("weight") is w and bufs.get("scales") is s and bufs.get("biases") is b:
+            # The usual call, checked again in native code (None: anything unusual, sorted out below).
+            y = linear(x, w, s, b, wp, sp, bp)
+            if type(y) is int:
+                _lib.check(y, "QuantizedLinear")
+            if y is not None:
+                return y
         if (mod.weight is not w or mod.scales is not s or mod.biases is not b or w.data_ptr() != wp
                 or s.data_ptr() != sp or b.data_ptr() != bp or s.dtype != torch.bfloat16
                 or b.dtype != torch.bfloat16):
@@ -174,7 +183,7 @@ def _launcher(mod: QuantizedLinear):
 
 def _call(self: QuantizedLinear, x: torch.Tensor) -> torch.Tensor:
     sh = x.shape
-    rows = math.prod(sh[:-1])
+    rows = sh[0] if len(sh) == 2 else math.prod(sh[:-1])
     if "_fast" not in self.__dict__ and not eligible(self):
         # packed_linear._call (84-86): a module the packed path does not take runs the general op
         # (here quantized_matmul's exact dequantize + bf16 GEMM form: 4-bit shapes the kernels

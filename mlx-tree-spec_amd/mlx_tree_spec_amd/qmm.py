@@ -112,6 +112,21 @@ def _general_kernel_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bo
     return not (x.requires_grad and torch.is_grad_enabled()) and torch.autograd.forward_ad._current_level < 0
 
 
+def _native_qmm(x, w, scales, biases, transpose, group_size, bits, mode):
+    """The usual call in native code (the output), or None for the general form below."""
+    if transpose is not True or mode != "affine" or not x.is_cuda or x.dim() < 1 or w.dim() != 2:
+        return None
+    k, n = x.shape[-1], w.shape[0]
+    general = bits != 4 or group_size != 64 or k % 128 != 0 or n % 16 != 0
+    if general and (bits not in GENERAL_BITS or group_size not in GENERAL_GROUP_SIZES or k == 0
+                    or not _general_kernel_ok(x, x.numel() // k, n, k, bits)):
+        return None
+    y = _lib.native().qmm(x, w, scales, biases, group_size, bits, general)
+    if type(y) is int:
+        _lib.check(y, "quantized_matmul")
+    return y
+
+
 def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases: torch.Tensor,
                      transpose: bool = True, group_size: int = 64, bits: int = 4,
                      mode: str = "affine") -> torch.Tensor:
@@ -124,6 +139,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     registers; others dequantize the weights and multiply by a bf16 GEMM, both with fp32
     accumulation on the same stream.
     """
+    y = _native_qmm(x, w, scales, biases, transpose, group_size, bits, mode)
+    if y is not None:
+        return y
     _check_format(group_size, bits, transpose, mode, general=True)
     if x.dtype != torch.bfloat16:
         raise ValueError(f"[quantized_matmul] x must be bfloat16, got {x.dtype}")
@@ -173,6 +191,12 @@ def gate_up_silu(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, biases:
     bf16(bf16(g * bf16(sigmoid(g))) * u) elementwise, the unfused composition of
     tree_verify.py:446's layer.mlp (down_proj(silu(gate_proj(x)) * up_proj(x))) up to down_proj.
     """
+    if bits == 4 and group_size == 64 and mode == "affine" and x.is_cuda:
+        y = _lib.native().gate_up(x, w, scales, biases)
+        if type(y) is int:
+            _lib.check(y, "gate_up_silu")
+        if y is not None:
+            return y
     _check_format(group_size, bits, True, mode)
     if x.dtype != torch.bfloat16:
         raise ValueError(f"[gate_up_silu] x must be bfloat16, got {x.dtype}")
