@@ -432,7 +432,8 @@ void gemm_kernel(GemmParams P) {
       // last), item-major per lane (16-byte stores).
       const uint32_t slot = (uint32_t)bid * 2u + (u == u0 ? 0u : 1u);
 #pragma unroll
-      for (int i = 0; i < I; ++i)
+      for (int i = 0; i < I; ++i) {
+        if (m0 + wm * C::WM + i * 32 >= P.M) continue;  // rows past M: never read back
 #pragma unroll
         for (int j = 0; j < J; ++j)
 #pragma unroll
@@ -442,6 +443,7 @@ void gemm_kernel(GemmParams P) {
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rp,
                                                    (slot * (uint32_t)C::kPartF4 + item) * 16u, 0, 0);
           }
+      }
     }
     u = e;
     __syncthreads();  // the next segment's prologue reuses the LDS stages (and the output tile)
@@ -451,26 +453,20 @@ void gemm_kernel(GemmParams P) {
 // Stream-K fix-up: the tiles split between workgroups, their partial sums added in K order (the
 // owners of a tile's units in increasing order; a tile is the last segment of its first owner
 // when that owner's range began in an earlier tile), one f32x4 item per thread, bf16 y.
+// A block works within one tile, so the owners and slots are uniform, and in 32 bits (launch_sk_reduce
+// checks the range): 64-bit divisions per thread and contributor took part of its time:
+// 203 x 5120 -> 17408 69.6 -> 68.0 us, 333 x 5120 -> 5120 42.4 -> 41.6, others within 1%.
 constexpr int kSkRedThreads = 256;
 template <int BM, int BN>
 __global__ __launch_bounds__(kSkRedThreads) void gemm_sk_reduce_kernel(GemmParams P, int G) {
   using C = GemmCfg<BM, BN>;
-  const long long it = (long long)blockIdx.x * kSkRedThreads + threadIdx.x;
-  const int t = (int)(it / C::kPartF4);
-  const int e = (int)(it - (long long)t * C::kPartF4);
-  if (t >= P.sk_tiles) return;
-  const long long tb = (long long)t * P.upt;
-  const int lo = sk_owner(tb, P.U, G), hi = sk_owner(tb + P.upt - 1, P.U, G);
+  static_assert(C::kPartF4 % kSkRedThreads == 0, "whole blocks per tile");
+  constexpr int kBlocks = C::kPartF4 / kSkRedThreads;  // blocks per tile
+  const int t = blockIdx.x / kBlocks;
+  const int e = (int)(blockIdx.x % kBlocks) * kSkRedThreads + (int)threadIdx.x;
+  const uint32_t U = (uint32_t)P.U, tb = (uint32_t)t * (uint32_t)P.upt, g = (uint32_t)G;
+  const uint32_t lo = ((tb + 1) * g + U - 1) / U - 1, hi = ((tb + (uint32_t)P.upt) * g + U - 1) / U - 1;  // sk_owner
   if (lo == hi) return;  // one workgroup ran the whole tile and wrote it
-  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-      P.part, 0, rsrc_bytes((unsigned long long)G * 2 * C::kPartF4 * 16), kBufferRsrcWord3);
-  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int c = lo; c <= hi; ++c) {
-    const uint32_t slot = (uint32_t)c * 2u + ((c == lo && sk_start(lo, P.U, G) < tb) ? 1u : 0u);
-    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                  rp, (slot * (uint32_t)C::kPartF4 + (uint32_t)e) * 16u, 0, 0));
-    sum[0] += v[0]; sum[1] += v[1]; sum[2] += v[2]; sum[3] += v[3];
-  }
   // Tile origin (the same grouped walk as the main kernel; a quarter of a 256 x 256 tile when the
   // split range is the quarters of a full-tile launch's last tiles).
   const int id = P.quarter ? P.tile0 + (t >> 2) : t, qq = P.quarter ? t & 3 : 0;
@@ -484,7 +480,19 @@ __global__ __launch_bounds__(kSkRedThreads) void gemm_sk_reduce_kernel(GemmParam
   int mi, ni;
   part_item_coords<C>(e, &mi, &ni);
   const int n = n0 + ni;
-  if (n >= P.N) return;
+  if (n >= P.N || m0 + mi >= P.M) return;
+  const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+      P.part, 0, rsrc_bytes((unsigned long long)G * 2 * C::kPartF4 * 16), kBufferRsrcWord3);
+  // Every contributor but the first begins with this tile (its slot 0); the first ends with it, which is
+  // its slot 0 too when its range begins here (sk_start(lo) >= tb).
+  const uint32_t first = lo * 2u + (lo * U / g < tb ? 1u : 0u);
+  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (uint32_t c = lo; c <= hi; ++c) {
+    const uint32_t slot = c == lo ? first : c * 2u;
+    const f32x4 v = __builtin_bit_cast(
+        f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, (uint32_t)e * 16u, (int)(slot * (uint32_t)(C::kPartF4 * 16)), 0));
+    sum[0] += v[0]; sum[1] += v[1]; sum[2] += v[2]; sum[3] += v[3];
+  }
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
       P.y, 0, rsrc_bytes((unsigned long long)P.M * P.N * 2), kBufferRsrcWord3);
 #pragma unroll
@@ -661,7 +669,8 @@ void gemm_ws_kernel(GemmParams P) {
         // last), item-major per lane, as gemm_kernel stores them.
         const uint32_t slot = (uint32_t)bid * 2u + (first ? 0u : 1u);
 #pragma unroll
-        for (int i = 0; i < I; ++i)
+        for (int i = 0; i < I; ++i) {
+          if (m0 + wm * C::WM + i * 32 >= P.M) continue;  // rows past M: never read back
 #pragma unroll
           for (int j = 0; j < J; ++j)
 #pragma unroll
@@ -671,6 +680,7 @@ void gemm_ws_kernel(GemmParams P) {
               __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rp,
                                                      (slot * (uint32_t)C::kPartF4 + item) * 16u, 0, 0);
             }
+        }
       }
       __syncthreads();
     });
@@ -783,9 +793,10 @@ hipError_t launch_ws(const GemmParams& P, int blocks, hipStream_t stream) {
 
 template <int BM, int BN>
 hipError_t launch_sk_reduce(const GemmParams& P, int G, hipStream_t stream) {
-  const long long items = (long long)P.sk_tiles * GemmCfg<BM, BN>::kPartF4;
-  hipLaunchKernelGGL((gemm_sk_reduce_kernel<BM, BN>), dim3((unsigned)((items + kSkRedThreads - 1) / kSkRedThreads)),
-                     dim3(kSkRedThreads), 0, stream, P, G);
+  // The kernel's 32-bit owner arithmetic: (U + 1) (G + 1) below 2^32.
+  if ((unsigned long long)(P.U + 1) * (unsigned long long)(G + 1) >= 1ULL << 32) return hipErrorInvalidValue;
+  const long long blocks = (long long)P.sk_tiles * (GemmCfg<BM, BN>::kPartF4 / kSkRedThreads);
+  hipLaunchKernelGGL((gemm_sk_reduce_kernel<BM, BN>), dim3((unsigned)blocks), dim3(kSkRedThreads), 0, stream, P, G);
   return hipGetLastError();
 }
 
