@@ -64,7 +64,9 @@ constexpr int kRsThreads = 64 * kRsWaves;
 // min(row, M - 1); output rows 4 g + r lie in lane group g, so a unit's sums live in the MP / 4
 // lane groups g < MP / 4.
 constexpr int kRsPF = 2;  // units in flight per wave
-constexpr int kRsXB = 4;  // x pieces per thread per staging batch
+// x pieces per thread per staging batch (a batch is a memory round trip): more than 4 rows have up to
+// 80 KB of x per workgroup, 10 pieces.
+constexpr int rs_xb(int MP) { return MP > 4 ? 10 : 4; }
 // SMALL plans: each wave holds at most kRsPF units for the whole launch, and all of x (at most
 // kRsSmallXP 16-byte pieces per thread, 80 KB) is loaded global -> LDS directly; OWN plans hold
 // at most as much x. (Allowing the whole LDS at 8 waves sent 9-16 rows over 65552-99984 columns
@@ -166,7 +168,7 @@ void rowsplit_kernel(RowSplitParams P) {
   static_assert(!OWN || (!FUSED && !KSPLIT && !SMALL && !NORM && !PAIR && V == 4), "own blocks: plain whole-K projections");
   static_assert(!NORM || (MP == 4 && MP % kRsNormRows == 0), "thread groups of 256 per normalised row");
   constexpr int G = MP / 4;  // lane groups holding output rows
-  typedef f32x4 RowSums[G];  // the sums of one output column over x rows 4 g + r
+  constexpr int kRsXB = rs_xb(MP);
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int S = P.Kp >> 7;  // super-steps per row in this workgroup's K slice
   const int SU = P.SU;
@@ -350,9 +352,12 @@ void rowsplit_kernel(RowSplitParams P) {
     bv[j] = load_scales<V>(rb, so, (kq >> 5) + st * 4 * V);
   };
   // The ring holds units in the order they were taken, so the first unit past the end ends it.
-  // Whole K: the ring's first fetches go out behind the x loads, before their stores. K slices
-  // (few units per workgroup): the x stores first, then the fetches (measured: the decode down
-  // projection M = 1 over 5120 x 17408 21.4 -> 20.1 us; with whole K, 27.4 -> 28.4 us the other way).
+  // Whole K, and more than 4 rows: the ring's first fetches go out behind the x loads, before their
+  // stores. K slices at up to 4 rows (few units per workgroup, x in several batches): the x stores
+  // first, then the fetches (measured: the decode down projection M = 1 over 5120 x 17408 21.4 ->
+  // 20.1 us; with whole K, 27.4 -> 28.4 us the other way; 7 x 10240 -> 5120 15.7 -> 14.4, 16 x 5120 ->
+  // 17408 20.0 -> 19.5 with the fetches first).
+  constexpr bool EARLY = !KSPLIT || MP > 4;
   // OWN: wave w takes the SU steps of blocks w, w + 16, ... in turn; q counts its units.
   const int own_nq = OWN && wave < P.RB ? (P.RB - wave + kRsWaves - 1) / kRsWaves * SU : 0;
   auto own_unit = [&](int q) { return q < own_nq ? (wave + kRsWaves * (q / SU)) * SU + q % SU : U; };
@@ -363,7 +368,7 @@ void rowsplit_kernel(RowSplitParams P) {
   }
   // Units (groups) handed out by the LDS counter after the ring's first fill.
   constexpr int kFirst = PAIR ? kRsWaves : kRsPF * kRsWaves;
-  if constexpr (!KSPLIT) {
+  if constexpr (EARLY) {
     fetch(0, ua);
     fetch(1, ub);
     __builtin_amdgcn_sched_barrier(0);
@@ -420,7 +425,7 @@ void rowsplit_kernel(RowSplitParams P) {
     if (tid == 0) *next = kFirst;
   }
   __syncthreads();
-  if constexpr (KSPLIT) {
+  if constexpr (!EARLY) {
     fetch(0, ua);
     fetch(1, ub);
     __builtin_amdgcn_sched_barrier(0);
@@ -599,54 +604,55 @@ void rowsplit_kernel(RowSplitParams P) {
 
   // y[m, col] = sum over the block's steps, in step order, of its unit slots; element r of a slot's
   // lane group g is x row 4 g + r. Fused: the same for the column's gate and up blocks, then
-  // silu * up.
+  // silu * up. One item per (column, lane group), neighbouring threads in neighbouring columns.
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
       P.y, 0, rsrc_bytes((unsigned long long)P.M * P.Nout * 2), kBufferRsrcWord3);
-  auto row_sum = [&](int lrow, RowSums& sum) __attribute__((always_inline)) {
+  auto row_sum = [&](int lrow, int gg) __attribute__((always_inline)) {
     const int b = lrow >> 4, nn = lrow & 15;
-#pragma unroll
-    for (int gg = 0; gg < G; ++gg) sum[gg] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int st = 0; st < SS; ++st) {
+      const f32x4 c = part[((b * SS + st) * G + gg) * 16 + nn];
+      sum[0] += c[0]; sum[1] += c[1]; sum[2] += c[2]; sum[3] += c[3];
+    }
+    return sum;
+  };
+  auto write = [&](int col, int gg, const f32x4& sum, const f32x4& sup) __attribute__((always_inline)) {
 #pragma unroll
-      for (int gg = 0; gg < G; ++gg) {
-        const f32x4 c = part[((b * SS + st) * G + gg) * 16 + nn];
-        sum[gg][0] += c[0]; sum[gg][1] += c[1]; sum[gg][2] += c[2]; sum[gg][3] += c[3];
+    for (int r = 0; r < 4; ++r) {
+      const int m = 4 * gg + r;
+      if (m < P.M) {
+        const uint32_t o = FUSED ? silu_mul_bf16(bf16_rne(sum[r]), bf16_rne(sup[r])) : bf16_rne(sum[r]);
+        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)o, ry, (uint32_t)(m * P.Nout + col) * 2u, 0, 0);
       }
     }
   };
-  auto write = [&](int col, const RowSums& sum, const RowSums& sup) __attribute__((always_inline)) {
-#pragma unroll
-    for (int m = 0; m < MP; ++m)
-      if (m < P.M) {
-        const float v = sum[m >> 2][m & 3];
-        const uint32_t o = FUSED ? silu_mul_bf16(bf16_rne(v), bf16_rne(sup[m >> 2][m & 3])) : bf16_rne(v);
-        __builtin_amdgcn_raw_buffer_store_b16((uint16_t)o, ry, (uint32_t)(m * P.Nout + col) * 2u, 0, 0);
-      }
-  };
   if constexpr (!KSPLIT) {
-    for (int c = tid; c < P.R; c += kRsThreads) {
+    for (int it = tid; it < P.R * G; it += kRsThreads) {
+      const int gg = G == 1 ? 0 : it / P.R, c = it - gg * P.R;
       const int col = r0 + c;
-      if (col >= r1) continue;
-      RowSums sum, sup;
-      row_sum(c, sum);
-      if (FUSED) row_sum(P.R + c, sup);
-      write(col, sum, sup);
+      if (col >= r1 || 4 * gg >= P.M) continue;
+      const f32x4 sum = row_sum(c, gg);
+      const f32x4 sup = FUSED ? row_sum(P.R + c, gg) : sum;
+      write(col, gg, sum, sup);
     }
     return;
   }
 
-  // K slices: store this workgroup's fp32 row sums, count in, and let the last workgroup of the
-  // column range add the slices in slice order (the same bits whichever arrives last).
+  // K slices: store this workgroup's fp32 row sums ([lane group][row], contiguous for neighbouring
+  // threads), count in, and let the last workgroup of the column range add the slices in slice order
+  // (the same bits whichever arrives last). One item per (row, lane group) and every slice's load in
+  // flight at once: with one thread per column walking the lane groups and slices in turn, the last
+  // 7 of 31 us of 13 rows over the fused 5120 -> 34816 were this merge (time stamps): with the x staging
+  // in one batch 31.4 -> 28.3 us, 13 / 16 x 5120 -> 17408 20.3 / 20.2 -> 19.4 / 19.5.
   const int RR = FUSED ? 2 * P.R : P.R;
   const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
       P.part, 0, rsrc_bytes((unsigned long long)gridDim.x * RR * G * 16), kBufferRsrcWord3);
-  for (int lrow = tid; lrow < RR; lrow += kRsThreads) {
-    RowSums sum;
-    row_sum(lrow, sum);
-#pragma unroll
-    for (int gg = 0; gg < G; ++gg)
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum[gg]), rp,
-                                             (((uint32_t)blockIdx.x * RR + lrow) * G + gg) * 16u, 0, kCoherent);
+  for (int it = tid; it < RR * G; it += kRsThreads) {
+    const int gg = G == 1 ? 0 : it / RR;
+    if (4 * gg >= P.M) continue;
+    const f32x4 sum = row_sum(it - gg * RR, gg);
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sum), rp,
+                                           ((uint32_t)blockIdx.x * (uint32_t)(RR * G) + (uint32_t)it) * 16u, 0, kCoherent);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -656,26 +662,30 @@ void rowsplit_kernel(RowSplitParams P) {
   }
   __syncthreads();
   if (*next == 0) return;
-  auto slice_sum = [&](int lrow, RowSums& sum) __attribute__((always_inline)) {
+  // Slices past the last read zero (an offset outside the buffer), and adding +0 leaves a sum that is
+  // not -0 unchanged (a sum from +0 never is -0).
+  constexpr int kMaxKS = MP == 8 ? 8 : 4;
+  for (int it = tid; it < P.R * G; it += kRsThreads) {
+    const int gg = G == 1 ? 0 : it / P.R, c = it - gg * P.R;
+    const int col = r0 + c;
+    if (col >= r1 || 4 * gg >= P.M) continue;
+    f32x4 v[kMaxKS], vu[FUSED ? kMaxKS : 1];
 #pragma unroll
-    for (int gg = 0; gg < G; ++gg) sum[gg] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int qq = 0; qq < P.KS; ++qq) {
+    for (int qq = 0; qq < kMaxKS; ++qq) {
+      const uint32_t o = qq < P.KS ? ((uint32_t)((range * P.KS + qq) * G + gg) * (uint32_t)RR + (uint32_t)c) * 16u : 0x80000000u;
+      v[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, kCoherent));
+      if constexpr (FUSED)
+        vu[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o + (uint32_t)P.R * 16u, 0, kCoherent));
+    }
+    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f}, sup = sum;
 #pragma unroll
-      for (int gg = 0; gg < G; ++gg) {
-        const f32x4 c = __builtin_bit_cast(
-            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, (((uint32_t)(range * P.KS + qq) * RR + lrow) * G + gg) * 16u,
-                                                         0, kCoherent));
-        sum[gg][0] += c[0]; sum[gg][1] += c[1]; sum[gg][2] += c[2]; sum[gg][3] += c[3];
+    for (int qq = 0; qq < kMaxKS; ++qq) {
+      sum[0] += v[qq][0]; sum[1] += v[qq][1]; sum[2] += v[qq][2]; sum[3] += v[qq][3];
+      if constexpr (FUSED) {
+        sup[0] += vu[qq][0]; sup[1] += vu[qq][1]; sup[2] += vu[qq][2]; sup[3] += vu[qq][3];
       }
     }
-  };
-  for (int c = tid; c < P.R; c += kRsThreads) {
-    const int col = r0 + c;
-    if (col >= r1) continue;
-    RowSums sum, sup;
-    slice_sum(c, sum);
-    if (FUSED) slice_sum(P.R + c, sup);
-    write(col, sum, sup);
+    write(col, gg, sum, sup);
   }
   if (tid == 0) __hip_atomic_store(&P.cnt[range], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
