@@ -198,7 +198,7 @@ void gemm_kernel(GemmParams P) {
   f32x16 acc[I][J];
 
   // One tile segment: K steps [kb, ke) of the tile at (m0, n0) into acc (kb and ke even; with
-  // SB8 multiples of 8).
+  // SB8 multiples of 8, or of 4 where D = 4).
   auto run_segment = [&](int m0, int n0, int kb, int ke) __attribute__((always_inline)) {
     const uint32_t xoff = (uint32_t)(m0 + a_r0) * (uint32_t)P.K * 2u + (uint32_t)a_kc * 16u;
     const uint32_t col = (uint32_t)(n0 + b_col);
@@ -229,7 +229,7 @@ void gemm_kernel(GemmParams P) {
     // written to LDS, snext the following block (loaded 3 steps before it is first needed).
     u32x4 scur = {0u, 0u, 0u, 0u}, bcur = scur, snext = scur, bnext = scur;
     auto load_sb8 = [&](int kt, u32x4& s8, u32x4& b8) __attribute__((always_inline)) {
-      const int k = kt < ke ? kt : kb;
+      const int k = kt < ke ? kt : (kb & ~7);
       s8 = __builtin_amdgcn_raw_buffer_load_b128(rs, soff, k * 2, 0);
       b8 = __builtin_amdgcn_raw_buffer_load_b128(rb, soff, k * 2, 0);
     };
@@ -339,7 +339,7 @@ void gemm_kernel(GemmParams P) {
     // Prologue: steps kb .. kb + D - 1 in registers, step kb in LDS, step kb + D in flight.
 #pragma unroll
     for (int i = 0; i < D; ++i) load(kb + i, raw[i]);
-    if constexpr (SB8) load_sb8(kb, scur, bcur);
+    if constexpr (SB8) load_sb8(kb & ~7, scur, bcur);
     {
       uint32_t sbits, bbits;
       sb_of(raw[0], kb, sbits, bbits);
@@ -358,13 +358,32 @@ void gemm_kernel(GemmParams P) {
     if constexpr (SB8) {
       // Unrolled by 8 (kb and ke are multiples of 8), so every step knows its group statically and
       // the next block's registers become the current ones by a plain copy at the end.
-      for (int kt = kb; kt < ke; kt += 8) {
+      int kt = kb;
+      if constexpr (D == 4) {
+        // Half units: a segment that starts in the middle of a block of 8 steps...
+        if (kb & 4) {
+          load_sb8(kb + 4, snext, bnext);
+          two(kt, std::integral_constant<int, 4>{});
+          two(kt + 2, std::integral_constant<int, 6>{});
+          scur = snext;
+          bcur = bnext;
+          kt += 4;
+        }
+      }
+      for (; kt + 8 <= ke; kt += 8) {
         two(kt, std::integral_constant<int, 0>{});
         two(kt + 2, std::integral_constant<int, 2>{});
         two(kt + 4, std::integral_constant<int, 4>{});
         two(kt + 6, std::integral_constant<int, 6>{});
         scur = snext;
         bcur = bnext;
+      }
+      if constexpr (D == 4) {
+        // ... or ends there.
+        if (kt < ke) {
+          two(kt, std::integral_constant<int, 0>{});
+          two(kt + 2, std::integral_constant<int, 2>{});
+        }
       }
     } else {
       for (int kt = kb; kt < ke; kt += 2) two(kt, std::integral_constant<int, 0>{});
@@ -952,6 +971,18 @@ bool gemm_plan(int M, int N, int K, int cus, size_t ws_capacity, const uint16_t*
   return true;
 }
 
+// Stream-K over 128-row tiles with 8-group scales: units of 4 K steps instead of 8 where they shorten the
+// longest range (U units over G workgroups leave at most half of them one unit more) and enough
+// workgroups have it. Units of 8 / 4: 203 / 256 / 128 x 5120 -> 17408 (1360 units over 256, 31% with a
+// sixth) 68.9 / 73.9 / 46.4 -> 65.8 / 70.7 / 44.8 us, 333 x 5120 -> 5120 (34%) 42.9 -> 40.2, 512 x 5120 ->
+// 1024 (25%) 22.4 -> 20.7; with few longer ranges the CUs that run them have the chip to themselves
+// (200 x 5120 -> 10240, 12%: 47.0 -> 47.8), and with more than half nothing is shorter (384 x 5120 ->
+// 17408 94.2 -> 95.1).
+static bool sk_half_units(long long U, int G) {
+  const long long rem = U % G;
+  return 5 * rem >= G && 2 * rem <= G;
+}
+
 hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
                        uint16_t* y, float* part, int M, int N, int K, int cus, hipStream_t stream) {
   GemmParams P;
@@ -982,7 +1013,7 @@ hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* 
     P.tile0 = 0;
     P.quarter = 0;
     P.sk = 1;
-    P.ups = sb8 ? 8 : 2;
+    P.ups = sb8 ? (sk_half_units((long long)P.tiles_m * P.tiles_n * (K / BK / 8), plan.G) ? 4 : 8) : 2;
     P.upt = K / BK / P.ups;
     P.sk_tiles = P.tiles_m * P.tiles_n;
     P.U = (long long)P.sk_tiles * P.upt;
