@@ -435,7 +435,7 @@ int dispatch_qmm(DeviceInfo* di, const void* x, const uint32_t* w, const void* s
   }
 
   // 9 to 16 rows over a small problem (at most 32 weight rows per CU, K <= 6144): the row-split
-  // kernel's form with x straight into registers, every load in flight from the start.
+  // kernel's form with one wave per K chunk, every load in flight from the start.
   RowSplitPlan rplan;
   if (M >= 9 && rowsplit_xreg_plan((int)M, (int)N, (int)K, di->cus, &rplan)) {
     e = launch_rowsplit(rplan, xb, w, sb, bb, yb, nullptr, nullptr, (int)M, (int)N, (int)K, stream);

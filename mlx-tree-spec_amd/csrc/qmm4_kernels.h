@@ -81,7 +81,7 @@ hipError_t launch_rowphase(const RowPhasePlan& plan, const uint16_t* x, const ui
 struct RowSplitPlan {
   int MP;       // x rows per A fragment (4 or 8)
   bool small;   // every unit in flight from the start, all of x in LDS, sums in registers
-  bool xreg;    // 9-16 rows over a small problem: x loaded straight into registers per K chunk
+  bool xreg;    // 9-16 rows over a small problem: one wave per K chunk, its x through LDS of its own
   bool pair;    // whole K with units taken in groups (consecutive steps of a block, one slot per group)
   int GU;       // units per group when pair
   bool own;     // whole K, each wave owning whole blocks with their sums in registers (no slots)
@@ -102,7 +102,7 @@ struct RowSplitPlan {
 // number of weight rows (for the fused gate+up, both halves).
 bool rowsplit_plan(int M, int N, int K, int cus, bool fused, RowSplitPlan* plan);
 // 9 to 16 rows over at most 32 weight rows per CU and K of at most 6144: one wave per 512-k chunk
-// of both of its workgroup's blocks, x loaded straight into registers.
+// of both of its workgroup's blocks, every load issued at the start.
 bool rowsplit_xreg_plan(int M, int N, int K, int cus, RowSplitPlan* plan);
 // The residual add + RMS norm folded into the row-split kernel's x staging: the projection's
 // input is n = rmsnorm(x + r) * weight over rows of K, and h = x + r and n are also stored.

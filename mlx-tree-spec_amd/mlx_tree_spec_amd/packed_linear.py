@@ -186,7 +186,7 @@ def _call(self: QuantizedLinear, x: torch.Tensor) -> torch.Tensor:
     rows = sh[0] if len(sh) == 2 else math.prod(sh[:-1])
     if "_fast" not in self.__dict__ and not eligible(self):
         # packed_linear._call (84-86): a module the packed path does not take runs the general op
-        # (here quantized_matmul's exact dequantize + bf16 GEMM form: 4-bit shapes the kernels
+        # (here quantized_matmul's general kernel or dequantize + bf16 GEMM form: 4-bit shapes the packed kernels
         # refuse, and 2-, 4- or 8-bit codes in groups of 32, 64 or 128; other widths raise
         # NotImplementedError).
         STATS["fallback"] += 1
