@@ -683,10 +683,12 @@ bool rowphase_plan(int M, int N, int K, int cus, RowPhasePlan* plan, bool fused)
   // 5120 -> 17408: 68 ranges x 3 slices (204 workgroups) took 31.0-32.0 us, 46 x 5 (230)
   // 28.1-28.7 us; 17408 -> 5120 ties and keeps 20 x 12 (14 x 18 of 3 blocks per wave: 16 / 48 /
   // 64 rows 22.6 / 30.9 / 32.3 -> 24.2 / 34.3 / 35.6 us). Ranges of one block per wave (twice the
-  // ranges, half the K slices, the same walk) when those ranges would leave a workgroup at most
-  // 3 phases, too few to pipeline: 32 / 64 x 5120 -> 5120 17.0 / 20.6 -> 16.0 / 19.4 us,
-  // 16 / 32 x 17408 -> 5120 24.8 / 27.9 -> 22.6 / 26.5 us; with 6 phases (64 x 17408 -> 5120)
-  // the doubled x reads cost more (33.5 -> 37.2 us). They also replace them when their walk is
+  // ranges, half the K slices and partial tiles, the same walk, x read twice as often) when those
+  // ranges would leave a workgroup at most 4 phases: 3 are too few to pipeline (32 / 64 x 5120 -> 5120
+  // 17.0 / 20.6 -> 16.0 / 19.4 us), and at 4 the halved partial tiles outweigh x, which is staged merged
+  // (33 / 64 / 96 x 8192 -> 8192 25.2 / 25.5 / 30.1 -> 21.7 / 22.3 / 27.4 us, 64 x 12288 -> 5120 23.5 -> 21.8, 64 x
+  // 16384 -> 4096 23.0 -> 21.3); with 5 or 6 phases it is even up to 64 rows (64 x 14336 / 17408 -> 5120) and
+  // slower past them (96 x 14336 / 17408 -> 5120 29.4 / 33.0 -> 30.5 / 34.8). They also replace them when their walk is
   // strictly shorter: 48 / 64 x 5120 -> 10240 (80 ranges x 3 slices, 7 phases, against 40 x 6 of
   // 4) 27.0 / 27.4 -> 24.3 / 26.2 us.
   auto narrow = [&](int c, int* phases) {
@@ -717,7 +719,7 @@ bool rowphase_plan(int M, int N, int K, int cus, RowPhasePlan* plan, bool fused)
     const int id1 = pick(1);
     if (id1 >= 0 && id1 != id) {
       const long long walk1 = narrow(id1, &ph1);
-      if (walk1 < walk || (walk1 == walk && ph <= 3)) id = id1;
+      if (walk1 < walk || (walk1 == walk && ph <= 4)) id = id1;
     }
   }
   if (id < 0) return false;
