@@ -36,6 +36,7 @@
 
 #include "qmm4_common.h"
 #include "qmm4_kernels.h"
+#include "qmm4_offsets.h"
 
 namespace qmm4 {
 
@@ -159,33 +160,32 @@ void rowphase_kernel(RowPhaseParams P) {
 
   // ---- staging of one phase's x pieces, global -> LDS directly (no registers) ----
   // Row-major: slot m * 16 V + c of the stage holds the 16-byte piece c ^ (m % 16) of row m's run of
-  // PH values (x[m][PH ph + 8 (c ^ (m % 16)) .. + 8)); rows m >= M lie past the resource and read as
-  // zero. Adjacent lanes thus read adjacent pieces of one row: the address unit merges the lanes of
-  // a load only where neighbouring lanes fall in one 64-byte segment (measured per CU on 1 KB loads
-  // that hit L2: 37 GB/s with 16 rows spread over neighbouring lanes, 86 GB/s with 4 or more lanes
-  // per row; into LDS 29 and 64 GB/s). The pieces used to lie in A-fragment order, one row per
-  // neighbouring lane; so (A/B, identical bits) 64 / 32 x 17408 -> 5120 31.8 / 25.0 -> 28.6 / 23.4 us,
-  // 112 x 5120 -> 17408 45.5 -> 38.4, 64 rows of the fused 5120 -> 34816 58.3 -> 47.1, 32 x 5120 ->
-  // 151936 (x is a sixth of its requests) within the spread. The XOR spreads the 16 rows that one
-  // fragment read touches (one piece each at the same place) over all banks. Wave w's j-th load
-  // fills slots j * kRpThreads + 64 w .. + 63, one contiguous kilobyte of the stage (the LDS
-  // destination of a lane is the instruction's base + 16 lane). Completion is waited for with an
-  // explicit vector memory count one phase later, before the barrier that publishes the stage.
-  constexpr int kXC = 16 * V;                // pieces per row and phase
-  constexpr int kXRows = kRpThreads / kXC;   // rows per load of the whole workgroup: 16 or 8
-  static_assert(C::kXPieces % kRpThreads == 0 && (kXRows == 16 || kXRows == 8), "whole x loads per thread");
+  // PH values (x[m][PH ph + 8 (c ^ (m % 16)) .. + 8)); rows m >= M lie past the resource by their lane
+  // offset (rowphase_x_offset) and read as zero. Adjacent lanes thus read adjacent pieces of one row:
+  // the address unit merges the lanes of a load only where neighbouring lanes fall in one 64-byte
+  // segment (measured per CU on 1 KB loads that hit L2: 37 GB/s with 16 rows spread over neighbouring
+  // lanes, 86 GB/s with 4 or more lanes per row; into LDS 29 and 64 GB/s). The pieces used to lie in
+  // A-fragment order, one row per neighbouring lane; so (A/B, identical bits) 64 / 32 x 17408 -> 5120
+  // 31.8 / 25.0 -> 28.6 / 23.4 us, 112 x 5120 -> 17408 45.5 -> 38.4, 64 rows of the fused 5120 ->
+  // 34816 58.3 -> 47.1, 32 x 5120 -> 151936 (x is a sixth of its requests) within the spread. The XOR
+  // spreads the 16 rows that one fragment read touches (one piece each at the same place) over all
+  // banks. Wave w's j-th load fills slots j * kRpThreads + 64 w .. + 63, one contiguous kilobyte of the
+  // stage (the LDS destination of a lane is the instruction's base + 16 lane). Completion is waited for
+  // with an explicit vector memory count one phase later, before the barrier that publishes the stage.
+  constexpr int kXC = 16 * V;  // pieces per row and phase
+  static_assert(C::kXPieces % kRpThreads == 0, "whole x loads per thread");
   typedef __attribute__((address_space(3))) void* lds_ptr;
-  const int xm = tid / kXC;
-  const uint32_t xo = ((uint32_t)xm * (uint32_t)P.K + (uint32_t)(8 * ((tid % kXC) ^ xm))) * 2u;
+  const uint32_t xo = rowphase_x_base<V, kRpThreads>(tid, P.K);
   auto stage_x = [&](int st, int ph, bool live) __attribute__((always_inline)) {
+    // The row steps are added at each load (opaque to the compiler): kept across phases they take up to
+    // 7 registers, and at 112 rows one is spilled, whose scratch traffic the explicit counts would miss.
+    uint32_t base = xo;
+    asm volatile("" : "+v"(base));
 #pragma unroll
     for (int j = 0; j < C::kXL; ++j) {
-      // Row xm + kXRows j: its offset is scalar, and so is its XOR where kXRows = 8 leaves bit 3 of
-      // the row to j (K % 512 == 0 and a phase is 512 or 1024 bytes, so bit 7 of the offset is c's).
-      const uint32_t off = live ? xo ^ (uint32_t)((j * kXRows & 8) * 16) : kOut;
+      const LoadOffset o = rowphase_x_offset<V, kRpThreads>(base, j, ph, P.K, live);
       const lds_ptr dst = (lds_ptr)(reinterpret_cast<uint8_t*>(xs(st)) + (size_t)(j * kRpThreads + 64 * wave) * 16);
-      const int so = ph * C::PH * 2 + j * kXRows * P.K * 2;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, dst, 16, off, so, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, dst, 16, o.lane, (int)o.scalar, 0, 0);
     }
   };
 
@@ -239,13 +239,13 @@ void rowphase_kernel(RowPhaseParams P) {
     wo[j] = (j < nbw) ? (uint32_t)grow(16 * (wave + kRpWaves * j) + n) * (uint32_t)(P.K >> 1) + (uint32_t)g * 16u : kOut;
   }
   // Piece v of every block of phase ph into register buffer J (a zero-length resource when the
-  // phase does not exist: the loads then read zero without touching memory).
+  // phase does not exist, and no scalar offset: the loads then read zero without touching memory).
   auto fetch_v = [&](int J, int v, int ph, bool live) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t*>(P.w), 0,
                                                                         live ? wrec : 0, kBufferRsrcWord3);
 #pragma unroll
     for (int j = 0; j < BPW; ++j)
-      wv[J][j][v] = __builtin_amdgcn_raw_buffer_load_b128(rw, wo[j] + (uint32_t)(v * 64), ph * (C::PH / 2), 0);
+      wv[J][j][v] = __builtin_amdgcn_raw_buffer_load_b128(rw, wo[j] + (uint32_t)(v * 64), live ? ph * (C::PH / 2) : 0, 0);
   };
 
   f32x4 acc[BPW][MB];
