@@ -39,4 +39,13 @@ __host__ __device__ inline LoadOffset rowphase_x_offset(uint32_t base, int j, in
   return {o + (uint32_t)(j * kRows) * (uint32_t)K * 2u, live ? (uint32_t)(ph * 256 * V) : 0u};
 }
 
+// General kernel, x in units of 64 k: load i takes 8 rows, lane / 8 the row and lane % 8 its 16-byte piece,
+// from row m0. Lane part of load i (x with 64 rows more below 2 GiB); u: the unit.
+__host__ __device__ inline uint32_t general_x_base(int m0, int lane, int K) {
+  return (uint32_t)(m0 + (lane >> 3)) * (uint32_t)K * 2u + (uint32_t)(lane & 7) * 16u;
+}
+__host__ __device__ inline LoadOffset general_x_offset(uint32_t base, int i, int u, int K, bool live) {
+  return {live ? base + (uint32_t)i * 16u * (uint32_t)K : 0x80000000u, live ? (uint32_t)(u * 128) : 0u};
+}
+
 }  // namespace qmm4

@@ -23,6 +23,7 @@
 // 8-bit 65.8 -> 16.8, 64 x 8192 -> 8191 8-bit 80.8 -> 28.5, 256 x 8192 -> 8191 8-bit 136.9 -> 90.4.
 #include "qmm4_common.h"
 #include "qmm4_kernels.h"
+#include "qmm4_offsets.h"
 
 namespace qmm4 {
 
@@ -103,7 +104,7 @@ void general_kernel(GeneralParams P) {
   const int wrow = P.K / 8 * BITS;  // bytes of a weight row
 
   // Rows past M, columns past N and groups past the last row lie past the end of their buffers (each
-  // below 2 GiB) and read as zero; kOut is past the end of all of them.
+  // below 2 GiB) by their lane offsets and read as zero; kOut is past the end of all of them.
   constexpr uint32_t kOut = 0x80000000u;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(P.x), 0, rsrc_bytes((unsigned long long)P.M * P.K * 2), kBufferRsrcWord3);
@@ -119,7 +120,7 @@ void general_kernel(GeneralParams P) {
 
   u32x4 xr[2][C::NX];
   Codes<BITS> wr[2][CB];
-  const uint32_t xo = (uint32_t)(m0 + (lane >> 3)) * (uint32_t)P.K * 2u + (uint32_t)(lane & 7) * 16u;
+  const uint32_t xo = general_x_base(m0, lane, P.K);
   auto load = [&](int j, int u) __attribute__((always_inline)) {
     const bool live = u < ue;
 #pragma unroll
@@ -131,8 +132,10 @@ void general_kernel(GeneralParams P) {
       if constexpr (BITS == 2) wr[j][c].v = __builtin_amdgcn_raw_buffer_load_b32(rw, o, so, 0);
     }
 #pragma unroll
-    for (int i = 0; i < C::NX; ++i)
-      xr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, live ? xo : kOut, live ? i * 16 * P.K + u * 128 : 0, 0);
+    for (int i = 0; i < C::NX; ++i) {
+      const LoadOffset xi = general_x_offset(xo, i, u, P.K, live);
+      xr[j][i] = __builtin_amdgcn_raw_buffer_load_b128(rx, xi.lane, (int)xi.scalar, 0);
+    }
   };
   // Scales and biases of the segment from unit u: groups g0 + lane % 4 + 4 j of row lane / 4.
   constexpr int kNL = kGnScMax / 4;

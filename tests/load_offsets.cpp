@@ -58,6 +58,23 @@ void rowphase_rows() {
   }
 }
 
+// The general kernel's x: MB row blocks of 16 from m0, units of 64 k and one past the slice's last.
+template <int MB>
+void general(int M, int K) {
+  const uint32_t size = (uint32_t)M * K * 2u;
+  for (int m0 = 0; m0 < M; m0 += 16 * MB)
+    for (int lane = 0; lane < 64; ++lane) {
+      const uint32_t base = general_x_base(m0, lane, K);
+      for (int i = 0; i < 2 * MB; ++i)
+        for (int u = 0; u <= K / 64; ++u) {
+          const int m = m0 + 8 * i + lane / 8;
+          const bool live = u < K / 64;
+          const long long want = live && m < M ? (long long)m * K * 2 + u * 128 + lane % 8 * 16 : -1;
+          check("general", general_x_offset(base, i, u, K, live), size, want, M, K, lane, i);
+        }
+    }
+}
+
 }  // namespace
 
 int main() {
@@ -70,6 +87,11 @@ int main() {
   rowphase_rows<96>();
   rowphase_rows<112>();
   rowphase_rows<128>();
+  for (int K : {64, 192, 2560}) {
+    for (int M : {1, 7, 8, 9, 16}) general<1>(M, K);
+    for (int M : {17, 24, 25, 32}) general<2>(M, K);
+    for (int M : {33, 64, 65, 100, 257}) general<4>(M, K);
+  }
   std::printf("loads checked: %lld, violations: %lld\n", g_checked, g_fail);
   return g_fail ? 1 : 0;
 }
