@@ -43,6 +43,7 @@
 
 #include "qmm4_common.h"
 #include "qmm4_kernels.h"
+#include "qmm4_offsets.h"
 
 namespace qmm4 {
 
@@ -186,11 +187,10 @@ void gemm_kernel(GemmParams P) {
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
       P.y, 0, rsrc_bytes((unsigned long long)P.M * P.N * 2), kBufferRsrcWord3);
 
-  // Loader roles. Activations: 16-byte chunk a_kc of rows a_r0 + 64 j (row j's offset goes in the
-  // scalar offset). Weights: words WPT * b_part .. + WPT - 1 of column n0 + b_col.
+  // Loader roles. Activations: 16-byte chunk a_kc of rows a_r0 + 64 j (the row in the lane offset, which
+  // is what bounds rows past M). Weights: words WPT * b_part .. + WPT - 1 of column n0 + b_col.
   const int a_kc = tid & 7;
   const int a_r0 = tid >> 3;
-  const int xrowp = C::RPP * P.K * 2;  // byte distance of consecutive load passes
   const int b_col = tid / C::TPC, b_part = tid % C::TPC;
   const int lrow = lane & 31;
   const int lk = (lane >> 5) * 8;
@@ -200,7 +200,7 @@ void gemm_kernel(GemmParams P) {
   // One tile segment: K steps [kb, ke) of the tile at (m0, n0) into acc (kb and ke even; with
   // SB8 multiples of 8, or of 4 where D = 4).
   auto run_segment = [&](int m0, int n0, int kb, int ke) __attribute__((always_inline)) {
-    const uint32_t xoff = (uint32_t)(m0 + a_r0) * (uint32_t)P.K * 2u + (uint32_t)a_kc * 16u;
+    const uint32_t xoff = gemm_x_base(m0, a_r0, P.K, a_kc);
     const uint32_t col = (uint32_t)(n0 + b_col);
     const uint32_t woff = col * (uint32_t)(P.K >> 1) + (uint32_t)(b_part * WPT * 4);
     const uint32_t soff = col * (uint32_t)(P.K >> 6) * 2u;
@@ -211,8 +211,10 @@ void gemm_kernel(GemmParams P) {
     auto load = [&](int kt, Raw<C>& R) {
       const int k = kt < ke ? kt : ke - 1;
 #pragma unroll
-      for (int j = 0; j < AJ; ++j)
-        R.a[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, k * BK * 2 + j * xrowp, 0);
+      for (int j = 0; j < AJ; ++j) {
+        const LoadOffset o = gemm_x_offset<C::RPP>(xoff, j, P.K, k);
+        R.a[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, o.lane, (int)o.scalar, 0);
+      }
       if constexpr (WPT >= 4) {
 #pragma unroll
         for (int v = 0; v < C::WV; ++v) R.w[v] = __builtin_amdgcn_raw_buffer_load_b128(rw, woff + v * 16, k * 32, 0);
@@ -709,7 +711,6 @@ void gemm_ws_kernel(GemmParams P) {
   // Producers.
   const int a_kc = pt & 7, a_r0 = pt >> 3;
   constexpr int kAJ = 8;  // activation chunks per thread and step (rows a_r0 + 32 j)
-  const int xrowp = 32 * P.K * 2;
   struct RawW {
     u32x4 a[kAJ];
     u32x4 w[2];
@@ -720,7 +721,7 @@ void gemm_ws_kernel(GemmParams P) {
     return (Gi & 1) ? (w >> 16) : (w & 0xFFFFu);
   };
   for_segments([&](int m0, int n0, int kb, int ke, bool) __attribute__((always_inline)) {
-    const uint32_t xoff = (uint32_t)(m0 + a_r0) * (uint32_t)P.K * 2u + (uint32_t)a_kc * 16u;
+    const uint32_t xoff = gemm_x_base(m0, a_r0, P.K, a_kc);
     const uint32_t col = (uint32_t)(n0 + pt);
     const uint32_t woff = col * (uint32_t)(P.K >> 1);
     const uint32_t soff = col * (uint32_t)(P.K >> 6) * 2u;
@@ -729,7 +730,10 @@ void gemm_ws_kernel(GemmParams P) {
     auto load = [&](int kt, RawW& R) __attribute__((always_inline)) {
       const int k = kt < ke ? kt : ke - 1;
 #pragma unroll
-      for (int j = 0; j < kAJ; ++j) R.a[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, k * BK * 2 + j * xrowp, 0);
+      for (int j = 0; j < kAJ; ++j) {
+        const LoadOffset o = gemm_x_offset<32>(xoff, j, P.K, k);
+        R.a[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, o.lane, (int)o.scalar, 0);
+      }
 #pragma unroll
       for (int v = 0; v < 2; ++v) R.w[v] = __builtin_amdgcn_raw_buffer_load_b128(rw, woff + v * 16, k * 32, 0);
     };

@@ -48,4 +48,14 @@ __host__ __device__ inline LoadOffset general_x_offset(uint32_t base, int i, int
   return {live ? base + (uint32_t)i * 16u * (uint32_t)K : 0x80000000u, live ? (uint32_t)(u * 128) : 0u};
 }
 
+// GEMM activations: load pass j of RPP rows each, row r0 + RPP j of the tile at row m0, 16-byte chunk kc of
+// K step kt (64 k). The lane part of pass 0, and the offset of pass j (x with 256 rows more below 4 GiB):
+__host__ __device__ inline uint32_t gemm_x_base(int m0, int r0, int K, int kc) {
+  return (uint32_t)(m0 + r0) * (uint32_t)K * 2u + (uint32_t)kc * 16u;
+}
+template <int RPP>
+__host__ __device__ inline LoadOffset gemm_x_offset(uint32_t base, int j, int K, int kt) {
+  return {base + (uint32_t)(j * RPP) * (uint32_t)K * 2u, (uint32_t)(kt * 128)};
+}
+
 }  // namespace qmm4

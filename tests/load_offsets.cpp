@@ -75,6 +75,21 @@ void general(int M, int K) {
     }
 }
 
+// The GEMM's activations: tiles of BM rows, RPP rows per load pass, K steps of 64.
+template <int BM, int RPP>
+void gemm(int M, int K) {
+  const uint32_t size = (uint32_t)M * K * 2u;
+  for (int m0 = 0; m0 < (M + 255) / 256 * 256; m0 += BM)  // quarters of a 256-row tile may lie past M whole
+    for (int r0 = 0; r0 < RPP; ++r0)
+      for (int kc = 0; kc < 8; ++kc)
+        for (int j = 0; j < BM / RPP; ++j)
+          for (int kt = 0; kt < K / 64; ++kt) {
+            const int m = m0 + r0 + RPP * j;
+            const long long want = m < M ? (long long)m * K * 2 + kt * 128 + kc * 16 : -1;
+            check("gemm", gemm_x_offset<RPP>(gemm_x_base(m0, r0, K, kc), j, K, kt), size, want, M, K, r0, j);
+          }
+}
+
 }  // namespace
 
 int main() {
@@ -92,6 +107,12 @@ int main() {
     for (int M : {17, 24, 25, 32}) general<2>(M, K);
     for (int M : {33, 64, 65, 100, 257}) general<4>(M, K);
   }
+  for (int K : {128, 1024})
+    for (int M : {65, 127, 128, 129, 203, 256, 300}) {
+      gemm<128, 64>(M, K);
+      gemm<256, 64>(M, K);
+      gemm<256, 32>(M, K);  // the role-split kernel
+    }
   std::printf("loads checked: %lld, violations: %lld\n", g_checked, g_fail);
   return g_fail ? 1 : 0;
 }
