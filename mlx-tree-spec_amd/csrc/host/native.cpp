@@ -235,4 +235,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__native(void) {
+  PyObject* m = PyModule_Create(&module);
+  // The torch this was built for (the loader refuses another: ATen's layouts are not stable).
+  if (m && PyModule_AddStringConstant(m, "TORCH_VERSION", QMM4_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -6,7 +6,9 @@ There is no fallback: if the library is missing or fails to load, every call rai
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libqmm4.so")
@@ -69,23 +71,37 @@ def load():
 _native = None
 
 
+class _NoNative:
+    """Stands in for the native module where it is not built or not for this torch and Python: every
+    function declines, so the Python form of each call runs."""
+
+    qmm = linear = gate_up = norm = norm_qmm = staticmethod(lambda *args: None)
+
+
 def native():
     """The native form of the package's calls (csrc/host/native.cpp), bound to the loaded library.
 
     Its functions take the usual call (plain contiguous aligned tensors on the current device) and
-    return None for anything else, or a negative error code of the library."""
+    return None for anything else, or a negative error code of the library. It is a fast path only: the
+    Python form behind it needs libqmm4.so alone."""
     global _native
     if _native is None:
         lib = load()
-        if not os.path.exists(os.path.join(_HERE, "_native.so")):
-            raise LibraryNotBuilt(f"{_HERE}/_native.so not found: build it with `python -m mlx_tree_spec_amd.build` "
-                                  "(or __graft_entry__.build())")
-        import torch  # noqa: F401  (its libraries are what the extension links to)
+        try:
+            import torch  # (its libraries are what the extension links to)
 
-        from . import _native as mod
-        mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
-            "qmm4_affine_bf16", "qmm4_gate_up_silu_bf16", "qmm_affine_general_bf16", "qmm4_add_rms_norm_bf16",
-            "qmm4_add_rms_norm_qmm_bf16")))
+            mod = importlib.import_module("._native", __package__)
+            built_for = getattr(mod, "TORCH_VERSION", "of another version")
+            if built_for != torch.__version__:
+                raise ImportError(f"built for torch {built_for}, this is {torch.__version__}")
+            mod.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+                "qmm4_affine_bf16", "qmm4_gate_up_silu_bf16", "qmm_affine_general_bf16", "qmm4_add_rms_norm_bf16",
+                "qmm4_add_rms_norm_qmm_bf16")))
+        except ImportError as e:
+            warnings.warn(f"mlx_tree_spec_amd: the native call path cannot be loaded ({e}); calls take their Python "
+                          "form, 6-13 us more host time each. Build it with `python -m mlx_tree_spec_amd.build`.",
+                          RuntimeWarning, stacklevel=2)
+            mod = _NoNative
         _native = mod
     return _native
 

@@ -2,8 +2,9 @@
 
     python -m mlx_tree_spec_amd.build      (with mlx-tree-spec_amd/ on sys.path)
 
-_native.so (csrc/host/, the calls of the package from tensors to the C ABI) is a CPython extension on
-libtorch, built with the host compiler.
+_native (csrc/host/, the calls of the package from tensors to the C ABI) is a CPython extension on
+libtorch, built with the host compiler. The package runs without it, with more host time per call: where
+it cannot be built, build() warns.
 
 Objects compile in parallel; the library is linked to a temporary name and renamed, so a reader
 never sees a half-written file.
@@ -17,6 +18,7 @@ import subprocess
 import sys
 import sysconfig
 import tempfile
+import warnings
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 PROJ_DIR = os.path.dirname(PKG_DIR)
@@ -30,7 +32,8 @@ LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
 FLOOR_DIR = os.path.join(CSRC, "floor")
 FLOOR_PATH = os.path.join(PKG_DIR, "libqmm4_floor.so")
 HOST_DIR = os.path.join(CSRC, "host")
-NATIVE_PATH = os.path.join(PKG_DIR, "_native.so")
+# Named for this Python, so that another one does not load it.
+NATIVE_PATH = os.path.join(PKG_DIR, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 ARCH = os.environ.get("QMM4_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops off: no v_pk_{add,mul,fma}_f32 in device code. hipcc's host pass warns that
@@ -74,6 +77,7 @@ def _build_native(out: str) -> None:
     lib = os.path.join(root, "lib")
     out_tmp = out + f".tmp{os.getpid()}"
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f'-DQMM4_TORCH_VERSION="{torch.__version__}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
            "-I", sysconfig.get_paths()["include"], "-I", os.path.join(root, "include"),
            "-I", os.path.join(root, "include", "torch", "csrc", "api", "include"),
@@ -90,10 +94,19 @@ def build(verbose: bool = False) -> str:
     with cf.ThreadPoolExecutor(max_workers=1) as ex:
         native = ex.submit(_build_native, NATIVE_PATH)
         _link(sources(), LIB_PATH)
-        native.result()
-    _link(sorted(os.path.join(FLOOR_DIR, f) for f in os.listdir(FLOOR_DIR) if f.endswith(".hip")), FLOOR_PATH)
+        _link(sorted(os.path.join(FLOOR_DIR, f) for f in os.listdir(FLOOR_DIR) if f.endswith(".hip")), FLOOR_PATH)
+        built = [LIB_PATH, FLOOR_PATH]
+        try:
+            native.result()
+            built.append(NATIVE_PATH)
+        except (ImportError, OSError, RuntimeError) as e:
+            # An extension of earlier sources must not stay behind: it would call the new library.
+            if os.path.exists(NATIVE_PATH):
+                os.remove(NATIVE_PATH)
+            warnings.warn(f"{NATIVE_PATH} could not be built; the package runs without it, with more host time "
+                          f"per call:\n{e}", RuntimeWarning, stacklevel=2)
     if verbose:
-        print(f"built {LIB_PATH}, {NATIVE_PATH} and {FLOOR_PATH}")
+        print("built " + ", ".join(built))
     return LIB_PATH
 
 
