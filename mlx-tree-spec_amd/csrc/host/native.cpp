@@ -13,6 +13,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -79,6 +81,13 @@ bool weights_match(const at::Tensor& w, const at::Tensor& s, const at::Tensor& b
          b.size(1) == k / group;
 }
 
+// Whether something sees or rewrites torch's own operations (same_current_device declines for dispatch
+// modes): the general path's library product is one of them, the kernel is not.
+bool observed() {
+  return at::impl::torch_function_mode_enabled() ||
+         (at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16);
+}
+
 PyObject* none() { Py_RETURN_NONE; }
 
 #define CALL(rc, expr)   \
@@ -97,7 +106,7 @@ PyObject* qmm(PyObject*, PyObject* const* a, Py_ssize_t na) {
   if (PyErr_Occurred()) return nullptr;
   const bool general = a[6] == Py_True;
   const int64_t k = x->sizes().back(), m = x->numel() / k, n = w->size(0);
-  if (group <= 0 || bits <= 0 || !weights_match(*w, *s, *b, k, group, bits)) return none();
+  if (group <= 0 || bits <= 0 || !weights_match(*w, *s, *b, k, group, bits) || (general && observed())) return none();
   at::Tensor y = empty_like_rows(*x, n);
   void* st = stream_of(*x);
   int rc;

@@ -18,6 +18,8 @@ asynchronously on the current stream of x's device.
 from __future__ import annotations
 
 import torch
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from . import _lib
 
@@ -99,7 +101,7 @@ GENERAL_KERNEL_MAX_ROWS = 256
 GENERAL_KERNEL_MAX_PRODUCT = 1 << 31
 
 
-def _general_kernel_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bool:
+def _general_shape_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bool:
     """Whether the general kernel takes this product: K a multiple of its 64-k unit, up to 256 rows or a
     small product, byte offsets (with up to 64 rows past the end) below 2 GiB, and no gradient asked
     of x (the library product is differentiable in x; the kernels are not)."""
@@ -112,6 +114,24 @@ def _general_kernel_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bo
     return not (x.requires_grad and torch.is_grad_enabled()) and torch.autograd.forward_ad._current_level < 0
 
 
+def _observed(x: torch.Tensor) -> bool:
+    """Whether something sees or rewrites torch's own operations on x, of which the general path's library
+    product is one: autocast to another type (its result then has that type), a tensor subclass, a function or
+    dispatch mode (the default device's own mode sees nothing of a product)."""
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
+        return True
+    if torch._C._len_torch_function_stack() > 0 and not all(
+            isinstance(mode, DeviceContext) for mode in _get_current_function_mode_stack()):
+        return True
+    return type(x) not in (torch.Tensor, torch.nn.Parameter) or torch._C._len_torch_dispatch_stack() > 0
+
+
+def _general_kernel_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bool:
+    """Whether quantized_matmul's general path is the general kernel: its rule on the product, and nothing that
+    would see the library product in its place."""
+    return not _observed(x) and _general_shape_ok(x, m, n, k, bits)
+
+
 def _native_qmm(x, w, scales, biases, transpose, group_size, bits, mode):
     """The usual call in native code (the output), or None for the general form below."""
     if transpose is not True or mode != "affine" or not x.is_cuda or x.dim() < 1 or w.dim() != 2:
@@ -119,8 +139,8 @@ def _native_qmm(x, w, scales, biases, transpose, group_size, bits, mode):
     k, n = x.shape[-1], w.shape[0]
     general = bits != 4 or group_size != 64 or k % 128 != 0 or n % 16 != 0
     if general and (bits not in GENERAL_BITS or group_size not in GENERAL_GROUP_SIZES or k == 0
-                    or not _general_kernel_ok(x, x.numel() // k, n, k, bits)):
-        return None
+                    or not _general_shape_ok(x, x.numel() // k, n, k, bits)):
+        return None  # (the native call looks for the rest of _general_kernel_ok itself)
     y = _lib.native().qmm(x, w, scales, biases, group_size, bits, general)
     if type(y) is int:
         _lib.check(y, "quantized_matmul")
@@ -136,8 +156,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
     them. Other shapes (K % 64 == 0, any N) and formats (2-, 4- or 8-bit codes in groups of 32, 64
     or 128) are what the reference leaves to MLX's own op (packed_linear.py:56-57, 84-86): up to 256
     rows (more over small weights; K % 64 == 0) run the general kernel, which dequantizes exactly in
-    registers; others dequantize the weights and multiply by a bf16 GEMM, both with fp32
-    accumulation on the same stream.
+    registers; others, and calls whose product something else sees (a gradient of x, autocast to another
+    type, function and dispatch modes), dequantize the weights and multiply by a bf16 GEMM, both
+    with fp32 accumulation on the same stream.
     """
     y = _native_qmm(x, w, scales, biases, transpose, group_size, bits, mode)
     if y is not None:

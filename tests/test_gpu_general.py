@@ -5,6 +5,7 @@ start inside a group of 128, and more than one scale segment (8 units) per wave.
 import numpy as np
 import pytest
 import torch
+from torch.utils.flop_counter import FlopCounterMode
 
 from mlx_tree_spec_amd import dequantize, quantized_matmul
 from mlx_tree_spec_amd.qmm import _general_kernel_ok
@@ -61,3 +62,38 @@ def test_general_path_keeps_the_gradient_of_x():
     want = wf.sum(0).expand(5, -1)
     # Sums of 33 bf16 weights rounded to bf16.
     assert torch.allclose(xd.grad.float(), want, rtol=2.0**-7, atol=1e-3)
+
+
+def test_general_path_shows_its_product_to_modes():
+    """Autocast to another type, function and dispatch modes and forward-mode derivatives see the general path's
+    product, in the native form of the call and behind it."""
+    x, w, s, b = _inputs(5, 256, 33, 8, 32, seed=4)
+    xd, wd = _dev(x, np.int16).view(torch.bfloat16), _dev(w, np.int32)
+    sd, bd = _dev(s, np.int16).view(torch.bfloat16), _dev(b, np.int16).view(torch.bfloat16)
+    call = lambda t: quantized_matmul(t, wd, sd, bd, group_size=32, bits=8)  # noqa: E731
+    wf = dequantize(wd, sd, bd, group_size=32, bits=8)
+    want = xd.float() @ wf.float().T.contiguous()
+    for dtype in (torch.float16, torch.float32, torch.bfloat16):
+        with torch.autocast("cuda", dtype):
+            y = call(xd)
+        assert y.dtype == dtype and torch.allclose(y.float(), want, rtol=2.0**-7, atol=2.0**-7 * want.abs().max())
+    seen = []
+
+    class Functions(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Functions():
+        call(xd)
+    assert torch.nn.functional.linear in seen
+    with FlopCounterMode(display=False) as flops:
+        call(xd)
+    assert flops.get_total_flops() == 2 * 5 * 256 * 33
+    sub = type("Sub", (torch.Tensor,), {})
+    assert type(call(xd.as_subclass(sub))) is sub
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(xd, torch.ones_like(xd))
+        tangent = torch.autograd.forward_ad.unpack_dual(call(dual)).tangent
+    # Sums of 256 bf16 weights rounded to bf16.
+    assert torch.allclose(tangent.float(), wf.float().sum(1).expand(5, -1), rtol=2.0**-7, atol=1e-3)
