@@ -94,18 +94,35 @@ def aligned_contiguous(t: torch.Tensor, align: int = 16) -> torch.Tensor:
 
 
 
-# The general kernel dequantizes the weights once per 64 rows, the other form once and runs a library
-# product: 256 x 8192 -> 8191 90 against 137 us, 512 rows 160 against 118; small products stay with the
-# kernel past 256 rows (512 x 1024 -> 513 6.7 against 29 us, 512 x 2560 -> 4101 41 against 34).
+# The general kernel dequantizes the weights once per 64 rows and has a fixed cost per 64 x 32 outputs; the other
+# form dequantizes once and runs a library product, at 38 us or more a call (the host's pace). Kernel / library
+# us, range over the 2-, 4- and 8-bit formats in groups of 32, 64 and 128: up to 32 rows the kernel wins everywhere
+# (at most 0.71 of the time, 32 x 256 -> 151937), up to 64, one pass over the weights, but over many columns of
+# little K (64 x 1024 -> 65537 46-50 / 61-77, but 48 x 256 -> 151937 60-63 / 48-56); two passes win from K = 4096 on
+# (128 x 5120 -> 17409 72-91 / 78-105, 128 x 4096 -> 65537 192-249 / 293-384, but 128 x 1024 -> 65537 84-88 / 68-84);
+# three and four up to 2^21 outputs (256 x 8192 -> 8191 84-98 / 95-111, 256 x 17408 -> 5121 133-163 / 209-248, but
+# 256 x 5120 -> 17409 126-157 / 101-140 and 160 x 4096 -> 11009 55-61 / 52-62) or with little work (160 x 512 ->
+# 16385 26 / 38). More than 256 rows: small products within the same lines (512 x 1024 -> 513 7 / 39, 2048 x 256 ->
+# 2047 27 / 38, but 4096 x 128 -> 4095 88 / 39, 262144 x 64 -> 127 162 / 56, 300 x 64 -> 65537 104 / 50).
 GENERAL_KERNEL_MAX_ROWS = 256
 GENERAL_KERNEL_MAX_PRODUCT = 1 << 31
 
 
+def _general_kernel_faster(m: int, n: int, k: int) -> bool:
+    if m <= 32:
+        return True
+    if m > GENERAL_KERNEL_MAX_ROWS and m * n * k > GENERAL_KERNEL_MAX_PRODUCT:
+        return False
+    outputs = (m + 63) // 64 * 64 * ((n + 31) // 32 * 32)  # of whole tiles
+    return (m <= 64 and k >= 1024 or m <= 128 and k >= 4096 or outputs <= 1 << 21
+            or outputs * (k + 512) <= 1 << 32)
+
+
 def _general_shape_ok(x: torch.Tensor, m: int, n: int, k: int, bits: int) -> bool:
-    """Whether the general kernel takes this product: K a multiple of its 64-k unit, up to 256 rows or a
-    small product, byte offsets (with up to 64 rows past the end) below 2 GiB, and no gradient asked
-    of x (the library product is differentiable in x; the kernels are not)."""
-    if k % 64 or m == 0 or n == 0 or not (m <= GENERAL_KERNEL_MAX_ROWS or m * n * k <= GENERAL_KERNEL_MAX_PRODUCT):
+    """Whether the general kernel takes this product: K a multiple of its 64-k unit, a size at which it is the
+    faster form, byte offsets (with up to 64 rows past the end) below 2 GiB, and no gradient asked of x
+    (the library product is differentiable in x; the kernels are not)."""
+    if k % 64 or m == 0 or n == 0 or not _general_kernel_faster(m, n, k):
         return False
     if (m + 64) * k * 2 >= 1 << 31 or (n + 64) * (k // 8 * bits) >= 1 << 31 or (n + 64) * (k // 32) * 2 >= 1 << 31:
         return False
@@ -154,9 +171,9 @@ def quantized_matmul(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor, bia
 
     Shapes the packed kernels take (4-bit codes in groups of 64, K % 128 == 0, N % 16 == 0) run
     them. Other shapes (K % 64 == 0, any N) and formats (2-, 4- or 8-bit codes in groups of 32, 64
-    or 128) are what the reference leaves to MLX's own op (packed_linear.py:56-57, 84-86): up to 256
-    rows (more over small weights; K % 64 == 0) run the general kernel, which dequantizes exactly in
-    registers; others, and calls whose product something else sees (a gradient of x, autocast to another
+    or 128) are what the reference leaves to MLX's own op (packed_linear.py:56-57, 84-86): K % 64 == 0 at the
+    sizes where it is faster (up to 32 rows, over most weights up to 256) run the general kernel, which
+    dequantizes exactly in registers; others, and calls whose product something else sees (a gradient of x, autocast to another
     type, function and dispatch modes), dequantize the weights and multiply by a bf16 GEMM, both
     with fp32 accumulation on the same stream.
     """

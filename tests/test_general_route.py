@@ -1,5 +1,5 @@
-"""Which calls of the general path stay with its library product (CPU only): those whose product something
-else sees. The general kernel would give autocast's result another type, leave no operation for a mode or a
+"""Which calls of the general path stay with its library product (CPU only): the sizes at which it is the faster
+form, and calls whose product something else sees. The general kernel would give autocast's result another type, leave no operation for a mode or a
 tensor subclass to see, and no gradient or tangent of x."""
 
 import contextlib
@@ -74,3 +74,24 @@ def test_forms_of_x():
     assert not taken(x)
     with torch.no_grad():
         assert taken(x)
+
+
+# Sizes at either side of the rule's lines, with the form that was measured as the faster one (us of the
+# kernel / the library product, 4-bit groups of 64).
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (32, 256, 151937, True),     # 30 / 48
+    (33, 256, 151937, False),    # 62 / 52 (groups of 32)
+    (33, 64, 65537, True),       # 23 / 37
+    (64, 1024, 65537, True), (65, 1024, 65537, False),
+    (128, 5120, 17409, True), (129, 5120, 17409, False), (256, 5120, 17409, False),  # 77 / 95, 103 / 109, 135 / 121
+    (256, 8192, 8191, True),     # 88 / 111
+    (160, 4096, 11009, False), (192, 512, 16385, True),
+    (256, 64, 65537, False),     # 85 / 38
+    (512, 1024, 513, True), (2048, 256, 2047, True), (400, 320, 16001, False), (300, 64, 65537, False),
+    (4096, 128, 4095, False),    # 88 / 42
+    (524288, 64, 3, False),      # 80 / 38
+    (320, 17408, 513, False),    # past 256 rows only small products
+])
+def test_sizes(m, k, n, kernel):
+    x = torch.empty((1, 1), dtype=torch.bfloat16).expand(m, k)
+    assert _general_kernel_ok(x, m, n, k, 4) is kernel
