@@ -86,3 +86,16 @@ def test_add_rms_norm_rejects_mismatched_shapes():
         add_rms_norm_(bf16_dev(x), bf16_dev(r), bf16_dev(w[:32]), 1e-6)
     with pytest.raises(ValueError):  # width not a multiple of 8
         add_rms_norm_(bf16_dev(x[:, :60]), bf16_dev(r[:, :60]), bf16_dev(w[:60]), 1e-6)
+
+
+# Either side of the lines between the two forms of the kernel (one or two chunks per thread: loads under a
+# branch, or all at the start), with whole waves and single threads past the row.
+@pytest.mark.parametrize("rows,d", [(7, 512), (3, 2048), (512, 2560), (513, 2560), (2252, 2560), (2253, 2560),
+                                    (600, 3072), (600, 3080), (4478, 1280), (4507, 1280), (4478, 1288)])
+def test_add_rms_norm_forms(rows, d):
+    x, r, w = inputs(rows, d, rows * 11 + d)
+    h, n = add_rms_norm_(bf16_dev(x), bf16_dev(r), bf16_dev(w), 1e-6)
+    ho, no = O.add_rms_norm(x, r, w, 1e-6)
+    nb = host_bits(n)
+    assert np.array_equal(host_bits(h), ho)
+    assert float(np.mean(nb == no)) >= 0.999 and within_ulps(nb, no, 2).all()
