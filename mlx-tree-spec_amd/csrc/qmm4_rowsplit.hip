@@ -65,8 +65,10 @@ constexpr int kRsThreads = 64 * kRsWaves;
 // lane groups g < MP / 4.
 constexpr int kRsPF = 2;  // units in flight per wave
 // x pieces per thread per staging batch (a batch is a memory round trip): more than 4 rows have up to
-// 80 KB of x per workgroup, 10 pieces.
-constexpr int rs_xb(int MP) { return MP > 4 ? 10 : 4; }
+// 80 KB of x per workgroup, 10 pieces. x of at most 4 pieces takes a batch of 4: surplus loads and stores
+// are not free (batches of 10 / 4: 9 x 512 -> 12288 5.47 / 4.84 us, 5 x 1024 -> 7168 5.68 / 5.01, 5 / 6 x 2560 ->
+// 5120 / 10240 7.23 / 11.1 against 6.59 / 10.6).
+constexpr int kRsFewX = 4, kRsMoreX = 10;
 // SMALL plans: each wave holds at most kRsPF units for the whole launch, and all of x (at most
 // kRsSmallXP 16-byte pieces per thread, 80 KB) is loaded global -> LDS directly; OWN plans hold
 // at most as much x. (Allowing the whole LDS at 8 waves sent 9-16 rows over 65552-99984 columns
@@ -134,8 +136,9 @@ __device__ __forceinline__ Scales<V> load_scales(__amdgpu_buffer_rsrc_t r, uint3
 // LDS accesses complete in order), but the compiler, which sees one lane, must keep the order too.
 __device__ __forceinline__ void wave_lds_order() { asm volatile("" ::: "memory"); }
 
-// Dynamic LDS: x pieces [16 S][MP] or [MP][16 S] (see the staging), unit slots [U][MP / 4][16] f32x4, a spare 16-byte slot (the target of surplus x pieces, so that every x store
-// is unconditional), the counter.
+// Dynamic LDS: x pieces [16 S][MP] or [MP][16 S] (see the staging), unit slots [U][MP / 4][16] f32x4, a
+// spare 16-byte slot (the target of surplus x pieces, so that every x store is unconditional), the
+// counter.
 __host__ __device__ inline size_t rowsplit_xs_bytes(int K, int MP) { return (size_t)(K >> 7) * 16 * MP * 16; }
 __host__ __device__ inline size_t rowsplit_part_bytes(int units, int MP) { return (size_t)units * (MP / 4) * 16 * 16; }
 
@@ -159,8 +162,13 @@ __host__ __device__ inline size_t rowsplit_red_offset(int Kp, int MP, int units,
 // is the bits of the unfused pair. Each workgroup reads all of x and r (from L2 after the first),
 // stages its K slice of n, and workgroup 0 writes h and n.
 // PAIR: 0, or units taken in groups: 1 for pairs, 2 for groups of P.GU > 2.
-template <int MP, int V, bool FUSED, bool KSPLIT, bool SMALL, bool NORM, int PAIR = 0, bool OWN = false>
-__global__ __launch_bounds__(kRsThreads) __attribute__((amdgpu_waves_per_eu(kRsWaves / 4)))
+// XB: x pieces per thread per staging batch. Small batches leave the compiler registers with which it aims
+// for more waves per SIMD than the one workgroup of a CU has, each LDS read then waited for before the next:
+// so the attribute ends at the workgroup's own waves there (6 rows of the fused 2048 -> 24576 / 1536 -> 65536
+// 10.9 / 16.3 -> 10.3 / 15.8 us).
+template <int MP, int V, bool FUSED, bool KSPLIT, bool SMALL, bool NORM, int PAIR, bool OWN, int XB>
+__global__ __launch_bounds__(kRsThreads)
+__attribute__((amdgpu_waves_per_eu(kRsWaves / 4, MP > 4 && XB == kRsFewX && !SMALL && !OWN ? kRsWaves / 4 : 8)))
 void rowsplit_kernel(RowSplitParams P) {
   static_assert(MP == 4 || MP == 8 || MP == 16, "x rows per fragment");
   static_assert(!SMALL || (!FUSED && !KSPLIT && !NORM), "small plans are plain whole-K projections of 6+ rows");
@@ -168,7 +176,6 @@ void rowsplit_kernel(RowSplitParams P) {
   static_assert(!OWN || (!FUSED && !KSPLIT && !SMALL && !NORM && !PAIR && V == 4), "own blocks: plain whole-K projections");
   static_assert(!NORM || (MP == 4 && MP % kRsNormRows == 0), "thread groups of 256 per normalised row");
   constexpr int G = MP / 4;  // lane groups holding output rows
-  constexpr int kRsXB = rs_xb(MP);
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   const int S = P.Kp >> 7;  // super-steps per row in this workgroup's K slice
   const int SU = P.SU;
@@ -210,11 +217,11 @@ void rowsplit_kernel(RowSplitParams P) {
   constexpr bool MERGE = MP > 4 && !ROWX;
   const int L = S * 16;
   const int xitems = L * P.M;
-  const int nxb = (xitems + kRsThreads * kRsXB - 1) / (kRsThreads * kRsXB);
+  const int nxb = (xitems + kRsThreads * XB - 1) / (kRsThreads * XB);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(P.x), 0, rsrc_bytes((unsigned long long)P.M * P.K * 2), kBufferRsrcWord3);
-  u32x4 xr[kRsXB];
-  int xp[kRsXB];  // MERGE: the LDS position of each item held in xr
+  u32x4 xr[XB];
+  int xp[XB];  // MERGE: the LDS position of each item held in xr
   // MERGE: row and piece of this thread's next item (items tid, tid + kRsThreads, ... in turn).
   int xm = 0, xq = 0, xdm = 0, xdq = 0;
   if constexpr (MERGE) {
@@ -225,7 +232,7 @@ void rowsplit_kernel(RowSplitParams P) {
   }
   auto load_x = [&](int batch) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kRsXB; ++j) {
+    for (int j = 0; j < XB; ++j) {
       uint32_t off;
       if constexpr (MERGE) {
         xp[j] = xm < P.M ? xq * MP + (xm ^ ((xq >> 2) & 3)) : (int)(spare - xs);
@@ -237,7 +244,7 @@ void rowsplit_kernel(RowSplitParams P) {
           ++xm;
         }
       } else {
-        const int i = tid + (batch * kRsXB + j) * kRsThreads;
+        const int i = tid + (batch * XB + j) * kRsThreads;
         const int sq = i / P.M, m = i - sq * P.M;
         off = i < xitems ? ((uint32_t)m * (uint32_t)P.K + (uint32_t)kq + (uint32_t)sq * 8u) * 2u : 0x80000000u;
       }
@@ -246,11 +253,11 @@ void rowsplit_kernel(RowSplitParams P) {
   };
   auto store_x = [&](int batch) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < kRsXB; ++j) {
+    for (int j = 0; j < XB; ++j) {
       if constexpr (MERGE) {
         xs[xp[j]] = xr[j];
       } else {
-        const int i = tid + (batch * kRsXB + j) * kRsThreads;
+        const int i = tid + (batch * XB + j) * kRsThreads;
         const int sq = i / P.M, m = i - sq * P.M;
         u32x4* dst = i < xitems ? xs + (sq * MP + m) : spare;
         *dst = xr[j];
@@ -1015,19 +1022,29 @@ size_t rowsplit_smem(const RowSplitPlan& plan, bool norm) {
                                  sizeof(float) * plan.MP * (kRsNormThreads / 64));
 }
 
-template <int MP, int V, bool FUSED, bool KSPLIT, bool SMALL, bool NORM, int PAIR = 0, bool OWN = false>
-hipError_t launch_rowsplit_t(const RowSplitPlan& plan, const RowSplitParams& P, hipStream_t stream) {
+template <int MP, int V, bool FUSED, bool KSPLIT, bool SMALL, bool NORM, int PAIR, bool OWN, int XB>
+hipError_t launch_rowsplit_xb(const RowSplitPlan& plan, const RowSplitParams& P, hipStream_t stream) {
   static bool attr_set = false;
   if (!attr_set) {
     hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN>),
+        reinterpret_cast<const void*>(&rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, XB>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRsLds);
     if (e != hipSuccess) return e;
     attr_set = true;
   }
-  hipLaunchKernelGGL((rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN>), dim3(plan.blocks),
+  hipLaunchKernelGGL((rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, XB>), dim3(plan.blocks),
                      dim3(kRsThreads), rowsplit_smem(plan, NORM), stream, P);
   return hipGetLastError();
+}
+
+template <int MP, int V, bool FUSED, bool KSPLIT, bool SMALL, bool NORM, int PAIR = 0, bool OWN = false>
+hipError_t launch_rowsplit_t(const RowSplitPlan& plan, const RowSplitParams& P, hipStream_t stream) {
+  // (SMALL, OWN and NORM do not stage x in batches.)
+  if constexpr (MP > 4 && !SMALL && !OWN && !NORM) {
+    if (P.M * (P.Kp >> 3) > kRsFewX * kRsThreads)
+      return launch_rowsplit_xb<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, kRsMoreX>(plan, P, stream);
+  }
+  return launch_rowsplit_xb<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, kRsFewX>(plan, P, stream);
 }
 
 template <int MP, int V, bool FUSED, bool NORM>

@@ -155,3 +155,12 @@ GEMM_STREAM_K_CASES = [
     (72, 65984, 2048, "128x256"),    # at most 128 rows over many columns: instead of whole tiles
     (96, 65984, 5120, "128x256"),
 ]
+
+# (M, K, N, gate+up, K slices) of row-split launches whose x takes M K / 8 / slices pieces of 16 bytes: at most 4 per
+# thread (2048) in one batch of 4, or batches of 10.
+ROWSPLIT_BATCH_CASES = [
+    (5, 512, 12288, False, 1), (8, 2048, 34816, False, 1), (7, 2560, 34816, False, 1), (9, 640, 8192, False, 1),
+    (16, 2048, 17408, False, 2), (16, 2560, 17408, False, 2), (6, 2560, 7168, False, 2), (8, 14336, 24576, False, 4),
+    (16, 14336, 5120, False, 4), (5, 512, 12288, True, 1), (8, 2560, 34816, True, 1), (13, 1280, 17408, True, 2),
+    (8, 8192, 34816, True, 2), (8, 5120, 151936, True, 8),
+]

@@ -221,3 +221,15 @@ def test_gemm_stream_k_cases_take_their_tiles(planner_exe):
     for (m, n, k, tiles), p in zip(GEMM_STREAM_K_CASES, query(planner_exe, lines)):
         assert p["sk"] == "1" and p["sk256"] == "0", (m, n, k, p)
         assert p["sk_wide"] == ("1" if tiles == "128x256" else "0"), (m, n, k, tiles, p)
+
+
+def test_rowsplit_batch_cases_take_their_slices(planner_exe):
+    """Each shape of test_gpu_rowsplit_batches.py is a row-split launch, staging x in batches, in the K slices that it
+    names."""
+    from route_cases import CUS, ROWSPLIT_BATCH_CASES
+
+    lines = [f"{'rowsplit_fused' if fused else 'rowsplit'} {m} {n} {k} {CUS}" for m, k, n, fused, _ in ROWSPLIT_BATCH_CASES]
+    for case, p in zip(ROWSPLIT_BATCH_CASES, query(planner_exe, lines)):
+        assert p["small"] == "0" and p["own"] == "0" and p["KS"] == str(case[4]), (case, p)
+    plain = [(m, n, k) for m, k, n, fused, _ in ROWSPLIT_BATCH_CASES if not fused]
+    assert dispatch_route(planner_exe, plain) == ["row-split"] * len(plain)
