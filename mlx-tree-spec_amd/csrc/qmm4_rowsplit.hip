@@ -107,6 +107,9 @@ struct RowSplitParams {
   float eps;
 };
 
+// The most K slices of a plan; the merge of a column range holds them all at once.
+constexpr int rs_max_ks(int MP) { return MP == 8 ? 8 : 4; }
+
 constexpr int kCoherent = 16;  // buffer access flag: bypass non-coherent caches (cross-CU partials)
 
 template <int V>
@@ -669,21 +672,34 @@ void rowsplit_kernel(RowSplitParams P) {
   }
   __syncthreads();
   if (*next == 0) return;
-  // Slices past the last read zero (an offset outside the buffer), and adding +0 leaves a sum that is
-  // not -0 unchanged (a sum from +0 never is -0).
-  constexpr int kMaxKS = MP == 8 ? 8 : 4;
+  // Slices past the last are +0, and adding +0 leaves a sum that is not -0 unchanged (a sum from +0 never
+  // is -0). KS is a power of 2, at most rs_max_ks(MP); loads of slices that are not there are not issued (6
+  // of 8 with 2 slices at 5-8 rows: 7 x 1024 -> 10240 8.4 -> 7.8 us, 6 x 2560 -> 7168 9.3 -> 8.9).
+  constexpr int kMaxKS = rs_max_ks(MP);
   for (int it = tid; it < P.R * G; it += kRsThreads) {
     const int gg = G == 1 ? 0 : it / P.R, c = it - gg * P.R;
     const int col = r0 + c;
     if (col >= r1 || 4 * gg >= P.M) continue;
     f32x4 v[kMaxKS], vu[FUSED ? kMaxKS : 1];
+    auto load_slices = [&](auto from, auto to, bool live) __attribute__((always_inline)) {
 #pragma unroll
-    for (int qq = 0; qq < kMaxKS; ++qq) {
-      const uint32_t o = qq < P.KS ? ((uint32_t)((range * P.KS + qq) * G + gg) * (uint32_t)RR + (uint32_t)c) * 16u : 0x80000000u;
-      v[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, kCoherent));
-      if constexpr (FUSED)
-        vu[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o + (uint32_t)P.R * 16u, 0, kCoherent));
-    }
+      for (int qq = decltype(from)::value; qq < decltype(to)::value; ++qq) {
+        v[qq] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (FUSED) vu[qq] = v[qq];
+      }
+      if (!live) return;
+#pragma unroll
+      for (int qq = decltype(from)::value; qq < decltype(to)::value; ++qq) {
+        const uint32_t o = ((uint32_t)((range * P.KS + qq) * G + gg) * (uint32_t)RR + (uint32_t)c) * 16u;
+        v[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, kCoherent));
+        if constexpr (FUSED)
+          vu[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o + (uint32_t)P.R * 16u, 0, kCoherent));
+      }
+    };
+    load_slices(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{}, true);
+    load_slices(std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{}, P.KS > 2);
+    if constexpr (kMaxKS > 4)
+      load_slices(std::integral_constant<int, 4>{}, std::integral_constant<int, 8>{}, P.KS > 4);
     f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f}, sup = sum;
 #pragma unroll
     for (int qq = 0; qq < kMaxKS; ++qq) {
@@ -939,7 +955,7 @@ bool rowsplit_plan(int M, int N, int K, int cus, bool fused, RowSplitPlan* plan)
   }
   // 9 to 16 rows: at most 4 K slices (x slices of 16 rows are large; with 8 slices, e.g. the
   // 65984-column head, the cross-workgroup merge of the slices costs more than it saves).
-  const int max_ks = MP == 8 ? 8 : 4;
+  const int max_ks = rs_max_ks(MP);
   const long long xbytes = (long long)M * K * 2;
   const long long wbytes = (long long)((nout + cus - 1) / cus) * (fused ? 2 : 1) * (K / 2);
   const int ks0 = (M >= 6 && 4 * xbytes > wbytes && K % 256 == 0) ? 2 : 1;
@@ -1094,7 +1110,7 @@ bool rowsplit_norm_ok(const RowSplitPlan& plan, int M, int K) {
 hipError_t launch_rowsplit(const RowSplitPlan& plan, const uint16_t* x, const uint32_t* w, const uint16_t* s,
                            const uint16_t* b, uint16_t* y, float* part, uint32_t* cnt, int M, int N, int K,
                            hipStream_t stream, const RowSplitNorm* norm) {
-  if (M > plan.MP) return hipErrorInvalidValue;
+  if (M > plan.MP || plan.KS > rs_max_ks(plan.MP)) return hipErrorInvalidValue;
   if (norm && !rowsplit_norm_ok(plan, M, K)) return hipErrorInvalidValue;
   RowSplitParams P;
   P.x = x; P.w = w; P.s = s; P.b = b; P.y = y;

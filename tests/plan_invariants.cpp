@@ -56,6 +56,7 @@ void check_rowsplit(int M, int N, int K, int cus, bool fused) {
   RS(p.fused == fused);
   RS(p.Nout == (fused ? N / 2 : N));
   RS(p.KS >= 1 && (long long)p.KS * p.Kp == K);
+  RS((p.KS & (p.KS - 1)) == 0);  // the merge loads 2, 4 or 8 slices
   RS(p.Kp % (128 * p.V) == 0);
   RS(p.SU == p.Kp / (128 * p.V) && p.SU >= 1);
   RS(p.R >= 4 && p.R % 4 == 0);
@@ -89,6 +90,19 @@ void check_rowsplit(int M, int N, int K, int cus, bool fused) {
     RS(p.smem == xs_bytes(p.Kp, p.MP) + part_bytes(p.RB * p.SU, p.MP) + 32);
   if (rowsplit_norm_ok(p, M, K)) RS(rowsplit_smem(p, true) <= kLds && M <= 4);
 #undef RS
+}
+
+// A plan of more K slices than the merge adds up is refused at the launch (before anything is launched).
+void check_slices_refused() {
+  for (int M : {1, 8, 16}) {
+    RowSplitPlan p{};
+    if (!rowsplit_plan(M, 17408, 5120, 256, false, &p)) continue;
+    ++g_checked;
+    p.KS = p.MP == 8 ? 16 : 8;
+    p.Kp = 5120 / p.KS;
+    CHECK(launch_rowsplit(p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, 17408, 5120, nullptr) ==
+              hipErrorInvalidValue, "rowsplit M=%d KS=%d", M, p.KS);
+  }
 }
 
 void check_xreg(int M, int N, int K, int cus) {
@@ -272,6 +286,7 @@ int main(int argc, char** argv) {
                     17408, 34816, 65984, 131072, 151936, 248320, 248336, 262144};
   const int Ks[] = {128, 256, 384, 512, 640, 1024, 2048, 2560, 4096, 5120, 6144, 8192, 12288, 17408, 20480};
   const int CUs[] = {256, 304, 80, 7, 1};
+  check_slices_refused();
   for (int cus : CUs)
     for (int M : Ms)
       for (int N : Ns)
