@@ -83,9 +83,9 @@ struct GemmParams {
 
 // Stream-K range of workgroup p: units [p U / G, (p + 1) U / G).
 __host__ __device__ inline long long sk_start(int p, long long U, int G) { return (long long)p * U / G; }
-// The workgroup whose range holds unit u.
-__host__ __device__ inline int sk_owner(long long u, long long U, int G) {
-  return (int)(((u + 1) * (long long)G + U - 1) / U) - 1;
+// The workgroup whose range holds unit u, in 32 bits ((U + 1) (G + 1) below 2^32).
+__host__ __device__ inline uint32_t sk_owner(uint32_t u, uint32_t U, uint32_t G) {
+  return ((u + 1) * G + U - 1) / U - 1;
 }
 
 template <int BM, int BN>
@@ -358,8 +358,8 @@ void gemm_kernel(GemmParams P) {
       step(kt + 1, std::integral_constant<int, 1>{}, std::integral_constant<int, U0 + 1>{});
     };
     if constexpr (SB8) {
-      // Unrolled by 8 (kb and ke are multiples of 8), so every step knows its group statically and
-      // the next block's registers become the current ones by a plain copy at the end.
+      // Unrolled by 8 from a multiple of 8, so every step knows its group statically and the next
+      // block's registers become the current ones by a plain copy at the end.
       int kt = kb;
       if constexpr (D == 4) {
         // Half units: a segment that starts in the middle of a block of 8 steps...
@@ -486,7 +486,7 @@ __global__ __launch_bounds__(kSkRedThreads) void gemm_sk_reduce_kernel(GemmParam
   const int t = blockIdx.x / kBlocks;
   const int e = (int)(blockIdx.x % kBlocks) * kSkRedThreads + (int)threadIdx.x;
   const uint32_t U = (uint32_t)P.U, tb = (uint32_t)t * (uint32_t)P.upt, g = (uint32_t)G;
-  const uint32_t lo = ((tb + 1) * g + U - 1) / U - 1, hi = ((tb + (uint32_t)P.upt) * g + U - 1) / U - 1;  // sk_owner
+  const uint32_t lo = sk_owner(tb, U, g), hi = sk_owner(tb + (uint32_t)P.upt - 1, U, g);
   if (lo == hi) return;  // one workgroup ran the whole tile and wrote it
   // Tile origin (the same grouped walk as the main kernel; a quarter of a 256 x 256 tile when the
   // split range is the quarters of a full-tile launch's last tiles).
@@ -864,6 +864,18 @@ int gemm_tail(int M, int N, int cus) {
   return (rem > 0 && 4 * rem <= 2 * c) ? rem : 0;
 }
 
+// Stream-K over 128-row tiles with 8-group scales: units of 4 K steps instead of 8 where they shorten the
+// longest range (U units over G workgroups leave at most half of them one unit more) and enough
+// workgroups have it. Units of 8 / 4: 203 / 256 / 128 x 5120 -> 17408 (1360 units over 256, 31% with a
+// sixth) 68.9 / 73.9 / 46.4 -> 65.8 / 70.7 / 44.8 us, 333 x 5120 -> 5120 (34%) 42.9 -> 40.2, 512 x 5120 ->
+// 1024 (25%) 22.4 -> 20.7; with few longer ranges the CUs that run them have the chip to themselves
+// (200 x 5120 -> 10240, 12%: 47.0 -> 47.8), and with more than half nothing is shorter (384 x 5120 ->
+// 17408 94.2 -> 95.1).
+bool sk_half_units(long long U, int G) {
+  const long long rem = U % G;
+  return 5 * rem >= G && 2 * rem <= G;
+}
+
 }  // namespace
 
 // More 128 x 128 tiles than CUs: whole rounds of 256 x 256 tiles (one per CU at a time) in one
@@ -879,6 +891,7 @@ bool gemm_plan(int M, int N, int K, int cus, size_t ws_capacity, const uint16_t*
   plan->sk_wide = false;
   plan->tail_sk = false;
   plan->G = 0;
+  plan->ups = 8;
   plan->part_bytes = 0;
   const long long tiles256 = (long long)((M + 255) / 256) * ((N + 255) / 256);
   // Stream-K over 256 x 256 tiles (one workgroup per CU, 8-step units): at least 256 rows, K of
@@ -971,20 +984,9 @@ bool gemm_plan(int M, int N, int K, int cus, size_t ws_capacity, const uint16_t*
   plan->sk = true;
   plan->sk_wide = wide;
   plan->G = (int)G;
+  plan->ups = sb8 ? (sk_half_units(U, (int)G) ? 4 : 8) : 2;
   plan->part_bytes = (size_t)G * slot;
   return true;
-}
-
-// Stream-K over 128-row tiles with 8-group scales: units of 4 K steps instead of 8 where they shorten the
-// longest range (U units over G workgroups leave at most half of them one unit more) and enough
-// workgroups have it. Units of 8 / 4: 203 / 256 / 128 x 5120 -> 17408 (1360 units over 256, 31% with a
-// sixth) 68.9 / 73.9 / 46.4 -> 65.8 / 70.7 / 44.8 us, 333 x 5120 -> 5120 (34%) 42.9 -> 40.2, 512 x 5120 ->
-// 1024 (25%) 22.4 -> 20.7; with few longer ranges the CUs that run them have the chip to themselves
-// (200 x 5120 -> 10240, 12%: 47.0 -> 47.8), and with more than half nothing is shorter (384 x 5120 ->
-// 17408 94.2 -> 95.1).
-static bool sk_half_units(long long U, int G) {
-  const long long rem = U % G;
-  return 5 * rem >= G && 2 * rem <= G;
 }
 
 hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b,
@@ -1002,7 +1004,7 @@ hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* 
     P.tile0 = 0;
     P.quarter = 0;
     P.sk = 1;
-    P.ups = 8;
+    P.ups = plan.ups;
     P.upt = K / BK / P.ups;
     P.sk_tiles = P.tiles_m * P.tiles_n;
     P.U = (long long)P.sk_tiles * P.upt;
@@ -1012,12 +1014,13 @@ hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* 
   }
   if (plan.sk) {
     if (plan.sk_wide && !sb8) return hipErrorInvalidValue;
+    if (plan.ups != 2 && !sb8) return hipErrorInvalidValue;
     P.tiles_m = (M + 127) / 128;
     P.tiles_n = plan.sk_wide ? (N + 255) / 256 : (N + 127) / 128;
     P.tile0 = 0;
     P.quarter = 0;
     P.sk = 1;
-    P.ups = sb8 ? (sk_half_units((long long)P.tiles_m * P.tiles_n * (K / BK / 8), plan.G) ? 4 : 8) : 2;
+    P.ups = plan.ups;
     P.upt = K / BK / P.ups;
     P.sk_tiles = P.tiles_m * P.tiles_n;
     P.U = (long long)P.sk_tiles * P.upt;
@@ -1047,7 +1050,7 @@ hipError_t launch_gemm(const GemmPlan& plan, const uint16_t* x, const uint32_t* 
     P.tile0 = main_tiles;
     P.quarter = 1;
     P.sk = 1;
-    P.ups = 8;
+    P.ups = plan.ups;
     P.upt = K / BK / P.ups;
     P.sk_tiles = 4 * tail;
     P.U = (long long)P.sk_tiles * P.upt;

@@ -143,6 +143,8 @@ struct GemmPlan {
   bool sk_wide;       // stream-K over 128 x 256 tiles
   bool tail_sk;       // whole tiles whose quarter-tile tail runs as stream-K over the quarters
   int G;              // stream-K workgroups (of the whole launch, or of the tail)
+  int ups;            // stream-K: K steps (64 k) per unit: 8, 4 where that shortens the longest range, or 2
+                      // without 8-group scale blocks
   size_t part_bytes;  // stream-K partial tiles (two per workgroup)
 };
 // `ws_capacity`: the most partial-tile bytes the caller's workspace can hold (stream-K spreads

@@ -4,6 +4,7 @@
 // the configurations their launch paths instantiate). Prints one line per violation and a summary;
 // the exit status is the number of violations (capped at 255). Built and run by
 // tests/test_plans.py; no GPU is touched.
+#include <algorithm>
 #include <cstdio>
 #include <cstdint>
 #include <string>
@@ -191,6 +192,9 @@ void check_gemm(int M, int N, int K, int cus) {
       const long long tiles = (long long)((M + tm - 1) / tm) * ((N + tn - 1) / tn);
       const long long units = tiles * (K / 64 / (K % 512 == 0 ? 8 : 2));
       GP(p.G >= 1 && p.G <= units);
+      GP(p.ups == 8 || (K % 512 == 0 ? p.ups == 4 && !p.sk256 : p.ups == 2));
+      // The fix-up's 32-bit owners, also with 2 workgroups per CU.
+      GP((unsigned long long)(tiles * (K / 64 / p.ups) + 1) * (unsigned long long)(2 * cus + 1) < 1ULL << 32);
       GP(p.part_bytes == (size_t)p.G * tm * tn * 4 * 2);
       GP(p.part_bytes <= cap);
       GP(!(p.sk256 && p.sk_wide));
@@ -201,7 +205,7 @@ void check_gemm(int M, int N, int K, int cus) {
       // Whole tiles whose last round (fewer quarters than CUs) runs as stream-K over its quarters.
       const long long total = (long long)((M + 255) / 256) * ((N + 255) / 256);
       const long long rem = total % cus;
-      GP(K % 512 == 0 && rem > 0 && 4 * rem < cus && !p.sk256);
+      GP(K % 512 == 0 && rem > 0 && 4 * rem < cus && !p.sk256 && p.ups == 8);
       GP(p.G >= 1 && p.G <= 4 * rem * (K / 512));
       GP(p.part_bytes == (size_t)p.G * 128 * 128 * 4 * 2 && p.part_bytes <= cap);
     } else {
@@ -248,8 +252,8 @@ int query() {
         std::printf("none\n");
         continue;
       }
-      std::printf("sk=%d sk256=%d sk_wide=%d tail_sk=%d G=%d\n", (int)p.sk, (int)p.sk256, (int)p.sk_wide,
-                  (int)p.tail_sk, p.G);
+      std::printf("sk=%d sk256=%d sk_wide=%d tail_sk=%d G=%d ups=%d\n", (int)p.sk, (int)p.sk256, (int)p.sk_wide,
+                  (int)p.tail_sk, p.G, p.ups);
     } else {
       std::printf("unknown\n");
     }
@@ -287,6 +291,13 @@ int main(int argc, char** argv) {
   const int Ks[] = {128, 256, 384, 512, 640, 1024, 2048, 2560, 4096, 5120, 6144, 8192, 12288, 17408, 20480};
   const int CUs[] = {256, 304, 80, 7, 1};
   check_slices_refused();
+  // The longest K that the 4 GiB limits on x and w leave the GEMM, over shapes of up to 512 tiles.
+  for (int M : {65, 128, 512, 1448, 2048, 4096})
+    for (int N : {16, 256, 2048, 4096, 5792, 8192}) {
+      const long long k = std::min((1LL << 31) / (M + 256), (1LL << 33) / (N + 256)) - 1;
+      check_gemm(M, N, (int)(k / 128 * 128), 256);
+      check_gemm(M, N, (int)(k / 512 * 512), 256);
+    }
   for (int cus : CUs)
     for (int M : Ms)
       for (int N : Ns)

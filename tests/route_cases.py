@@ -164,3 +164,8 @@ ROWSPLIT_BATCH_CASES = [
     (16, 14336, 5120, False, 4), (5, 512, 12288, True, 1), (8, 2560, 34816, True, 1), (13, 1280, 17408, True, 2),
     (8, 8192, 34816, True, 2), (8, 5120, 151936, True, 8),
 ]
+
+# (M, K, N, 128 x 256 tiles) of stream-K launches in units of 4 K steps. U units of 8 steps over 256 workgroups:
+# 640 (128 x 128 tiles, half the ranges longer), 320 (a quarter), 1360 (128 x 256 tiles, 203 rows: the last
+# row of tiles partly past M).
+GEMM_HALF_UNIT_CASES = [(129, 2048, 10240, False), (512, 5120, 1024, False), (203, 5120, 17408, True)]

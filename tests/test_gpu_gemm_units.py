@@ -1,19 +1,19 @@
 """Stream-K GEMM launches in units of 4 K steps: workgroup ranges that start and end in the middle of a
-block of 8 scales, over 128 x 128 and 128 x 256 tiles, and with scales outside the fast form's range."""
+block of 8 scales, over 128 x 128 and 128 x 256 tiles, and with scales outside the fast form's range
+(test_plans.py checks that the shapes take those units)."""
 
 import pytest
 import torch
 
 from mlx_tree_spec_amd import dequantize, quantized_matmul
+from route_cases import GEMM_HALF_UNIT_CASES
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("big_scale", [False, True])
-# U units of 8 steps over 256 workgroups: 640 (128 x 128 tiles, half the ranges longer), 320 (a
-# quarter), 1360 (128 x 256 tiles, 203 rows: the last row of tiles partly past M).
-@pytest.mark.parametrize("m,k,n", [(129, 2048, 10240), (512, 5120, 1024), (203, 5120, 17408)])
+@pytest.mark.parametrize("m,k,n", [case[:3] for case in GEMM_HALF_UNIT_CASES])
 def test_half_unit_ranges(m, k, n, big_scale):
     g = torch.Generator(device=DEV).manual_seed(m + k + n)
     x = torch.randn(m, k, generator=g, device=DEV).bfloat16()

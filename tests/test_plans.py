@@ -233,3 +233,16 @@ def test_rowsplit_batch_cases_take_their_slices(planner_exe):
         assert p["small"] == "0" and p["own"] == "0" and p["KS"] == str(case[4]), (case, p)
     plain = [(m, n, k) for m, k, n, fused, _ in ROWSPLIT_BATCH_CASES if not fused]
     assert dispatch_route(planner_exe, plain) == ["row-split"] * len(plain)
+
+
+def test_half_unit_cases_take_units_of_4(planner_exe):
+    """The shapes of test_gpu_gemm_units.py are stream-K launches in units of 4 K steps, over the tiles it names;
+    neighbours past either end of the rule (an eighth of the ranges longer, or more than half) take 8."""
+    from route_cases import CUS, GEMM_HALF_UNIT_CASES
+
+    cases = [(m, n, k, wide, "4") for m, k, n, wide in GEMM_HALF_UNIT_CASES]
+    cases += [(200, 10240, 5120, True, "8"), (384, 17408, 5120, True, "8"), (136, 5120, 640, False, "2")]
+    out = query(planner_exe, [f"gemm {m} {n} {k} {CUS}" for m, n, k, _, _ in cases])
+    for (m, n, k, wide, ups), p in zip(cases, out):
+        assert p["sk"] == "1" and p["sk256"] == "0" and p["ups"] == ups, (m, n, k, p)
+        assert p["sk_wide"] == str(int(wide)), (m, n, k, p)
