@@ -20,10 +20,11 @@
 //    so each row is read as one contiguous run per unit. Rows past the workgroup's range read as
 //    zero (an offset outside the buffer resource), as do fetches past the last unit (a zero-length
 //    resource).
-//  * x (M <= MP rows, MP = 4, 8 or 16, whole K or the workgroup's K slice) is staged once in LDS in
-//    A-fragment order. Every wave issues its x loads before any wave issues a weight fetch (a bare
-//    barrier between the two), and the stores wait for the x loads alone (the vector memory
-//    counter is in order).
+//  * x (M <= MP rows, MP = 4, 8 or 16, whole K or the workgroup's K slice) is staged once in LDS, in
+//    A-fragment order (past 4 rows with the rows of a piece swizzled), or row by row in the SMALL and
+//    OWN forms. Every wave issues its x loads before any wave issues a weight fetch (a bare
+//    barrier between the two; SMALL and OWN the other way round), and the stores wait for the x loads
+//    alone (the vector memory counter is in order).
 //  * Dequantization: dequant_word_fast, or dequant_word for a unit in which one of the wave's
 //    rows has a scale outside the fast form's range (a wave-uniform branch per unit).
 //  * Each unit's fp32 sums (MFMA 16x16x32, bf16 inputs; output row 4 g + r in lane group g) go to
@@ -693,7 +694,8 @@ void rowsplit_kernel(RowSplitParams P) {
         const uint32_t o = ((uint32_t)((range * P.KS + qq) * G + gg) * (uint32_t)RR + (uint32_t)c) * 16u;
         v[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o, 0, kCoherent));
         if constexpr (FUSED)
-          vu[qq] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o + (uint32_t)P.R * 16u, 0, kCoherent));
+          vu[qq] = __builtin_bit_cast(
+              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, o + (uint32_t)P.R * 16u, 0, kCoherent));
       }
     };
     load_slices(std::integral_constant<int, 0>{}, std::integral_constant<int, 2>{}, true);

@@ -131,6 +131,10 @@ ROWPHASE_WIDE_CASES = [
 ROWPHASE_SHAPES = [(17, 5120, 4096), (33, 2048, 32784), (9, 5120, 65984), (48, 3072, 33024), (64, 1024, 2064),
                    (24, 17408, 1024), (16, 5120, 65984), (32, 2048, 65984), (16, 5120, 99984), (32, 2048, 131072),
                    (24, 5120, 17408), (12, 17408, 5120), (48, 6144, 5120), (32, 2048, 8192)]
+# (M, K, N, blocks per range) of narrow plans around the line of 4 phases per workgroup: ranges of one block per
+# wave (8) where two (16) would leave at most 4, ranges of two at 5 phases and more.
+ROWPHASE_PHASE_CASES = [(33, 8192, 8192, 8), (96, 8192, 8192, 8), (64, 12288, 5120, 8), (64, 16384, 4096, 8),
+                        (80, 7680, 8192, 8), (112, 4096, 14336, 8), (64, 14336, 5120, 16), (96, 17408, 5120, 16)]
 # (N, M, K) of the one-hot exact-dequantization test.
 ROWPHASE_ONE_HOT = [(32800, 32, 2048), (2064, 48, 2048), (65984, 16, 5120), (131072, 32, 2048), (4096, 80, 2048),
                     (2064, 112, 2048), (1024, 128, 2048), (33024, 48, 2048), (65984, 32, 2048), (65984, 64, 2048),

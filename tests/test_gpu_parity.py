@@ -22,8 +22,8 @@ import golden_io
 from mlx_tree_spec_amd import STATS, QuantizedLinear, dequantize, install, quantized_matmul
 from oracle import cpu
 from oracle import qmm4_oracle as O
-from route_cases import (MID_ROW_CASES, ROWPHASE_ONE_HOT, ROWPHASE_SHAPES, ROWPHASE_WIDE_CASES,
-                         ROWPHASE_WINDOW_CASES)
+from route_cases import (MID_ROW_CASES, ROWPHASE_ONE_HOT, ROWPHASE_PHASE_CASES, ROWPHASE_SHAPES,
+                         ROWPHASE_WIDE_CASES, ROWPHASE_WINDOW_CASES)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -717,11 +717,19 @@ def test_rowsplit_xreg_one_hot_is_exact_dequant(kind):
 # K = 3072 ends in a partial scale window. 65984 columns (the drafter's head) give a workgroup 17
 # blocks (the 3-blocks-per-wave variants), 99984 and 131072 columns 25 and 32 blocks (4 per wave).
 # 24 rows over 5120 -> 17408: K split over ranges of 3 blocks per wave (46 ranges x 5 slices).
-# Ranges of one block per wave where two would leave a workgroup at most 3 phases: 12 x 17408 ->
+# Ranges of one block per wave where two would leave a workgroup at most 4 phases: 12 x 17408 ->
 # 5120 (40 ranges x 6 slices of 6 phases), 48 x 6144 -> 5120 (4 phases), 32 x 2048 -> 8192.
 @pytest.mark.parametrize("m,k,n", ROWPHASE_SHAPES)
 def test_rowphase_shapes(m, k, n):
     note(f"row-phase {m}x{k}x{n}")
+    x, w, s, b = O.make_inputs(m, k, n, seed=m * 11 + k + n)
+    check_qmm(gpu_qmm(x, w, s, b), workload_ref(x, w, s, b), f"row-phase {m}x{k}x{n}", (x, w, s, b))
+
+
+# Narrow plans at either side of 4 phases per workgroup (tests/test_plans.py checks the ranges).
+@pytest.mark.parametrize("m,k,n,blocks", ROWPHASE_PHASE_CASES)
+def test_rowphase_phase_lines(m, k, n, blocks):
+    note(f"row-phase {m}x{k}x{n} ({blocks} blocks per range)")
     x, w, s, b = O.make_inputs(m, k, n, seed=m * 11 + k + n)
     check_qmm(gpu_qmm(x, w, s, b), workload_ref(x, w, s, b), f"row-phase {m}x{k}x{n}", (x, w, s, b))
 

@@ -246,3 +246,15 @@ def test_half_unit_cases_take_units_of_4(planner_exe):
     for (m, n, k, wide, ups), p in zip(cases, out):
         assert p["sk"] == "1" and p["sk256"] == "0" and p["ups"] == ups, (m, n, k, p)
         assert p["sk_wide"] == str(int(wide)), (m, n, k, p)
+
+
+def test_rowphase_ranges_at_the_line_of_4_phases(planner_exe):
+    """The shapes of test_gpu_parity.py's phase lines are row-phase launches with K split, in ranges of the blocks that
+    they name."""
+    from route_cases import CUS, ROWPHASE_PHASE_CASES
+
+    out = query(planner_exe, [f"rowphase {m} {n} {k} {CUS}" for m, k, n, _ in ROWPHASE_PHASE_CASES])
+    for case, p in zip(ROWPHASE_PHASE_CASES, out):
+        assert p["wide"] == "0" and p["BW"] == str(case[3]), (case, p)
+    routes = dispatch_route(planner_exe, [(m, n, k) for m, k, n, _ in ROWPHASE_PHASE_CASES])
+    assert routes == ["row-phase"] * len(routes)
