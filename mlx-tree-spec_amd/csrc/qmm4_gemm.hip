@@ -43,6 +43,7 @@
 
 #include "qmm4_common.h"
 #include "qmm4_kernels.h"
+#include "qmm4_lds.h"
 #include "qmm4_offsets.h"
 
 namespace qmm4 {
@@ -528,13 +529,9 @@ __global__ __launch_bounds__(kSkRedThreads) void gemm_sk_reduce_kernel(GemmParam
 template <int BM, int BN, bool SB8, int D = 2>
 hipError_t launch_tiles(const GemmParams& P, int blocks, hipStream_t stream) {
   constexpr size_t smem = GemmCfg<BM, BN>::kSmem;
-  static bool attr_set = false;  // the attribute is per function; setting it twice is harmless
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_kernel<BM, BN, SB8, D>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsAllowance lds;
+  const hipError_t e = lds.allow(reinterpret_cast<const void*>(&gemm_kernel<BM, BN, SB8, D>), smem);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL((gemm_kernel<BM, BN, SB8, D>), dim3(blocks), dim3(kThreads), smem, stream, P);
   return hipGetLastError();
 }
@@ -803,13 +800,9 @@ void gemm_ws_kernel(GemmParams P) {
 
 hipError_t launch_ws(const GemmParams& P, int blocks, hipStream_t stream) {
   constexpr size_t smem = GemmCfg<256, 256>::kSmem;
-  static bool attr_set = false;  // the attribute is per function; setting it twice is harmless
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_ws_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsAllowance lds;
+  const hipError_t e = lds.allow(reinterpret_cast<const void*>(&gemm_ws_kernel), smem);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(gemm_ws_kernel, dim3(blocks), dim3(kWsThreads), smem, stream, P);
   return hipGetLastError();
 }

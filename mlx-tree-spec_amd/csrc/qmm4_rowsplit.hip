@@ -49,6 +49,7 @@
 
 #include "qmm4_common.h"
 #include "qmm4_kernels.h"
+#include "qmm4_lds.h"
 
 namespace qmm4 {
 
@@ -1042,14 +1043,10 @@ size_t rowsplit_smem(const RowSplitPlan& plan, bool norm) {
 
 template <int MP, int V, bool FUSED, bool KSPLIT, bool SMALL, bool NORM, int PAIR, bool OWN, int XB>
 hipError_t launch_rowsplit_xb(const RowSplitPlan& plan, const RowSplitParams& P, hipStream_t stream) {
-  static bool attr_set = false;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, XB>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRsLds);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsAllowance lds;
+  const hipError_t e = lds.allow(
+      reinterpret_cast<const void*>(&rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, XB>), kRsLds);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL((rowsplit_kernel<MP, V, FUSED, KSPLIT, SMALL, NORM, PAIR, OWN, XB>), dim3(plan.blocks),
                      dim3(kRsThreads), rowsplit_smem(plan, NORM), stream, P);
   return hipGetLastError();
@@ -1092,13 +1089,9 @@ hipError_t launch_rowsplit_m(const RowSplitPlan& plan, const RowSplitParams& P, 
 }
 
 hipError_t launch_rowsplit_xreg(const RowSplitPlan& plan, const RowSplitParams& P, hipStream_t stream) {
-  static bool attr_set = false;  // the attribute is per function; setting it twice is harmless
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&rowsplit_xreg_kernel),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRsLds);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
+  static LdsAllowance lds;
+  const hipError_t e = lds.allow(reinterpret_cast<const void*>(&rowsplit_xreg_kernel), kRsLds);
+  if (e != hipSuccess) return e;
   hipLaunchKernelGGL(rowsplit_xreg_kernel, dim3(plan.blocks), dim3(64 * plan.SU),
                      plan.smem + (size_t)plan.SU * (kXrHalf + kXrSc), stream, P);
   return hipGetLastError();

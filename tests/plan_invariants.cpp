@@ -10,6 +10,7 @@
 #include <string>
 
 #include "qmm4_kernels.h"
+#include "qmm4_lds.h"
 
 namespace qmm4 {
 // Defined in qmm4_rowsplit.hip (exported, not in the kernels header): the plan's dynamic LDS, with
@@ -104,6 +105,20 @@ void check_slices_refused() {
     CHECK(launch_rowsplit(p, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, M, 17408, 5120, nullptr) ==
               hipErrorInvalidValue, "rowsplit M=%d KS=%d", M, p.KS);
   }
+}
+
+// Large dynamic LDS is allowed once on every device, and again where that failed.
+void check_lds_allowance() {
+  LdsAllowance a;
+  int calls = 0;
+  auto set = [&](hipError_t e) { return [&calls, e] { ++calls; return e; }; };
+  ++g_checked;
+  const bool ok = a.once(0, set(hipErrorInvalidValue)) == hipErrorInvalidValue && a.once(0, set(hipSuccess)) == hipSuccess &&
+                  a.once(0, set(hipErrorInvalidValue)) == hipSuccess && calls == 2 &&
+                  a.once(1, set(hipSuccess)) == hipSuccess && calls == 3 && a.once(63, set(hipSuccess)) == hipSuccess &&
+                  a.once(1, set(hipErrorInvalidValue)) == hipSuccess && calls == 4 &&
+                  a.once(64, set(hipSuccess)) == hipSuccess && a.once(64, set(hipSuccess)) == hipSuccess && calls == 6;
+  CHECK(ok, "lds allowance after %d calls", calls);
 }
 
 void check_xreg(int M, int N, int K, int cus) {
@@ -291,6 +306,7 @@ int main(int argc, char** argv) {
   const int Ks[] = {128, 256, 384, 512, 640, 1024, 2048, 2560, 4096, 5120, 6144, 8192, 12288, 17408, 20480};
   const int CUs[] = {256, 304, 80, 7, 1};
   check_slices_refused();
+  check_lds_allowance();
   // The longest K that the 4 GiB limits on x and w leave the GEMM, over shapes of up to 512 tiles.
   for (int M : {65, 128, 512, 1448, 2048, 4096})
     for (int N : {16, 256, 2048, 4096, 5792, 8192}) {
