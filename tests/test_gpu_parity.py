@@ -599,7 +599,7 @@ def test_rowsplit_eight_row_shapes(m, k, n):
         assert np.array_equal(host_bits(quantized_matmul(xd, wd, sd, bd)), y)
 
 
-# 9 to 16 rows beyond the x-in-registers form's reach: the row-split kernel with 16-row fragments,
+# 9 to 16 rows beyond the one-wave-per-chunk form's reach: the row-split kernel with 16-row fragments,
 # x in LDS in up to 4 K slices (the MLP up projection at 9 and 16 rows: 2 slices; 12 rows over
 # 34816 columns: 2 slices of 5-step units; K = 2048 over 16384 columns: the small form; K = 6144).
 @pytest.mark.parametrize("m,k,n", [(9, 5120, 17408), (16, 5120, 17408), (12, 5120, 34816), (16, 5120, 10240),
@@ -673,13 +673,13 @@ def test_rowsplit_small_and_eight_row_one_hot_is_exact_dequant(kind, m, n):
         assert not bad.any(), f"{int(bad.sum())} mismatches at k0={k0}, first {np.argwhere(bad)[:3].tolist()}"
 
 
-# 9 to 16 rows over at most 32 weight rows per CU with K <= 6144: the row-split form with x loaded
-# straight into registers, one wave per 512-k chunk. 16 x 5120 over 5120 columns (c0: 20 rows per
+# 9 to 16 rows over at most 32 weight rows per CU with K <= 6144: the row-split form with one wave per
+# 512-k chunk, its x in order through the wave's own LDS. 16 x 5120 over 5120 columns (c0: 20 rows per
 # workgroup, a half-live second block), 12 rows over 2048 (8 rows per workgroup), N = 8208 (a partial
-# last range), 9 rows (fragment rows 9-15 repeat row 8).
+# last range), 9 rows (fragment rows 9-15 are zero).
 @pytest.mark.parametrize("m,k,n", [(16, 5120, 5120), (12, 4096, 2048), (16, 2048, 8208), (9, 5120, 1024)])
 def test_rowsplit_xreg_shapes(m, k, n):
-    note(f"row-split x-in-registers {m}x{k}x{n}")
+    note(f"row-split one-wave-per-chunk {m}x{k}x{n}")
     x, w, s, b = O.make_inputs(m, k, n, seed=m * 23 + k + n)
     xd, wd, sd, bd = bf16_dev(x), u32_dev(w), bf16_dev(s), bf16_dev(b)
     y = host_bits(quantized_matmul(xd, wd, sd, bd))
@@ -689,7 +689,7 @@ def test_rowsplit_xreg_shapes(m, k, n):
 
 @pytest.mark.parametrize("kind", ["fast", "mixed", "slow"])
 def test_rowsplit_xreg_one_hot_is_exact_dequant(kind):
-    """One-hot rows of x through the x-in-registers form: single dequantized weights, bit for bit."""
+    """One-hot rows of x through the one-wave-per-chunk form: single dequantized weights, bit for bit."""
     m, k, n = 16, 5120, 5120
     rng = np.random.default_rng({"fast": 41, "mixed": 42, "slow": 43}[kind])
     s, b = scale_bias_pairs(kind, n * (k // 64), rng)

@@ -1,7 +1,7 @@
 """Kernel planners against what their kernels assume (CPU only, no GPU call).
 
 tests/plan_invariants.cpp calls the planners exported by the built libqmm4.so (row-split, its
-x-in-registers form, row-phase, K-split verify, GEMM) over a grid of shapes (1-4096 rows, 16-262144 columns,
+one-wave-per-chunk form, row-phase, K-split verify, GEMM) over a grid of shapes (1-4096 rows, 16-262144 columns,
 K = 128-20480) and CU counts (1-304), and checks every accepted plan: dynamic LDS within 160 KB,
 output columns covered exactly once, K slices and units that tile K, each loop form only in the
 configuration its launch path instantiates, stream-K workgroups between 1 and the unit count
@@ -98,7 +98,7 @@ def test_random_gate_up_shapes_reach_every_route(planner_exe):
 def gate_up_routes(planner_exe, shapes):
     """dispatch_gate_up_silu's route for each (M, K, N) on 256 CUs, from the planners' answers: the
     fused row-split launch; else the row-phase plan the projection would take (5-96 rows, K % 512 ==
-    0, no row-split or x-in-registers plan up to 16 rows), fused: a wide plan under the range-size
+    0, no row-split or one-wave-per-chunk plan up to 16 rows), fused: a wide plan under the range-size
     rule, a narrow (K-split) plan where the projection takes it (17 rows or more, or a K split
     filling half the CUs); else the two passes."""
     from route_cases import CUS
@@ -175,7 +175,7 @@ def dispatch_route(exe, cases):
     """dispatch_qmm's route for each (M, N, K) on 256 CUs with 16-byte aligned scales, from the
     built planners queried in dispatch order: past 64 rows the row-phase kernel (narrow plans up to
     112 rows or 128 over at most 2048 columns, wide plans of at most one range per CU up to 96
-    rows) else the GEMM; up to 64 rows the x-in-registers row-split form (9-16 rows), the row-split
+    rows) else the GEMM; up to 64 rows the one-wave-per-chunk row-split form (9-16 rows), the row-split
     kernel, the row-phase kernel (from 5 rows when its plan is wide, has 17+ rows or fills half the
     CUs), else the verify or skinny kernel ("other")."""
     from route_cases import CUS
