@@ -64,6 +64,15 @@ void* stream_of(const at::Tensor& x) {
 }
 
 void* ptr(const at::Tensor& t) { return const_cast<void*>(t.const_data_ptr()); }
+// A new output's data, or null where a transform hands out a wrapper without storage of its own.
+void* out_ptr(const at::Tensor& t) { return t.has_storage() && t.is_cuda() ? ptr(t) : nullptr; }
+
+struct Weights {
+  const uint32_t* w;
+  const void *s, *b;
+  Weights(const at::Tensor& codes, const at::Tensor& scales, const at::Tensor& biases)
+      : w(static_cast<const uint32_t*>(ptr(codes))), s(ptr(scales)), b(ptr(biases)) {}
+};
 
 bool is_codes(const at::Tensor& w) { return w.dim() == 2 && (w.scalar_type() == at::kInt || w.scalar_type() == at::kUInt32); }
 bool is_bf16(const at::Tensor& t) { return t.scalar_type() == at::kBFloat16; }
@@ -90,6 +99,7 @@ bool observed() {
 
 PyObject* none() { Py_RETURN_NONE; }
 
+// `expr` runs without the GIL: it touches no tensor and throws nothing (pointers are taken before).
 #define CALL(rc, expr)   \
   Py_BEGIN_ALLOW_THREADS \
   rc = (expr);           \
@@ -108,14 +118,14 @@ PyObject* qmm(PyObject*, PyObject* const* a, Py_ssize_t na) {
   const int64_t k = x->sizes().back(), m = x->numel() / k, n = w->size(0);
   if (group <= 0 || bits <= 0 || !weights_match(*w, *s, *b, k, group, bits) || (general && observed())) return none();
   at::Tensor y = empty_like_rows(*x, n);
-  void* st = stream_of(*x);
+  const Weights q(*w, *s, *b);
+  void *st = stream_of(*x), *xp = ptr(*x), *yp = out_ptr(y);
+  if (!yp) return none();
   int rc;
   if (general) {
-    CALL(rc, p_general(ptr(*x), static_cast<const uint32_t*>(ptr(*w)), ptr(*s), ptr(*b), ptr(y), m, n, k, (int)group,
-                       (int)bits, st))
+    CALL(rc, p_general(xp, q.w, q.s, q.b, yp, m, n, k, (int)group, (int)bits, st))
   } else {
-    CALL(rc, p_affine(ptr(*x), static_cast<const uint32_t*>(ptr(*w)), ptr(*s), ptr(*b), ptr(y), m, n, k, (int)group,
-                      (int)bits, 1, st))
+    CALL(rc, p_affine(xp, q.w, q.s, q.b, yp, m, n, k, (int)group, (int)bits, 1, st))
   }
   return rc == 0 ? THPVariable_Wrap(std::move(y)) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
@@ -133,9 +143,11 @@ PyObject* linear(PyObject*, PyObject* const* a, Py_ssize_t na) {
   const int64_t k = x->sizes().back(), m = x->numel() / k, n = w->size(0);
   if (!weights_match(*w, *s, *b, k, 64, 4)) return none();
   at::Tensor y = empty_like_rows(*x, n);
-  void* st = stream_of(*x);
+  const Weights q(*w, *s, *b);
+  void *st = stream_of(*x), *xp = ptr(*x), *yp = out_ptr(y);
+  if (!yp) return none();
   int rc;
-  CALL(rc, p_affine(ptr(*x), static_cast<const uint32_t*>(ptr(*w)), ptr(*s), ptr(*b), ptr(y), m, n, k, 64, 4, 1, st))
+  CALL(rc, p_affine(xp, q.w, q.s, q.b, yp, m, n, k, 64, 4, 1, st))
   return rc == 0 ? THPVariable_Wrap(std::move(y)) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -149,9 +161,11 @@ PyObject* gate_up(PyObject*, PyObject* const* a, Py_ssize_t na) {
   const int64_t k = x->sizes().back(), m = x->numel() / k, n = w->size(0);
   if (n % 32 != 0 || !weights_match(*w, *s, *b, k, 64, 4)) return none();
   at::Tensor y = empty_like_rows(*x, n / 2);
-  void* st = stream_of(*x);
+  const Weights q(*w, *s, *b);
+  void *st = stream_of(*x), *xp = ptr(*x), *yp = out_ptr(y);
+  if (!yp) return none();
   int rc;
-  CALL(rc, p_gate_up(ptr(*x), static_cast<const uint32_t*>(ptr(*w)), ptr(*s), ptr(*b), ptr(y), m, n, k, 64, 4, 1, st))
+  CALL(rc, p_gate_up(xp, q.w, q.s, q.b, yp, m, n, k, 64, 4, 1, st))
   return rc == 0 ? THPVariable_Wrap(std::move(y)) : PyLong_FromLong(rc);
   END_HANDLE_TH_ERRORS
 }
@@ -170,10 +184,11 @@ PyObject* norm(PyObject*, PyObject* const* a, Py_ssize_t na) {
   if (!norm_args(x, r, w) || !same_current_device(*x, {r, w})) return none();
   const int64_t d = x->sizes().back(), m = x->numel() / d;
   at::Tensor h = at::empty(x->sizes(), x->options()), n = at::empty(x->sizes(), x->options());
-  void* st = stream_of(*x);
+  void *st = stream_of(*x), *xp = ptr(*x), *rp = ptr(*r), *wp = ptr(*w), *hp = out_ptr(h), *np = out_ptr(n);
+  if (!hp || !np) return none();
   const float eps = (float)PyFloat_AS_DOUBLE(a[3]);
   int rc;
-  CALL(rc, p_norm(ptr(*x), ptr(*r), ptr(*w), ptr(h), ptr(n), m, d, eps, st))
+  CALL(rc, p_norm(xp, rp, wp, hp, np, m, d, eps, st))
   if (rc != 0) return PyLong_FromLong(rc);
   PyObject* out = PyTuple_New(2);
   if (!out) return nullptr;
@@ -195,11 +210,14 @@ PyObject* norm_qmm(PyObject*, PyObject* const* a, Py_ssize_t na) {
   if ((silu && n % 32 != 0) || !weights_match(*w, *s, *b, k, 64, 4)) return none();
   at::Tensor h = at::empty(x->sizes(), x->options()), nn = at::empty(x->sizes(), x->options());
   at::Tensor y = empty_like_rows(*x, silu ? n / 2 : n);
-  void* st = stream_of(*x);
+  const Weights q(*w, *s, *b);
+  void *st = stream_of(*x), *xp = ptr(*x), *rp = ptr(*r), *np = ptr(*nw);
+  void *hp = out_ptr(h), *nnp = out_ptr(nn), *yp = out_ptr(y);
+  if (!hp || !nnp || !yp) return none();
   const float eps = (float)PyFloat_AS_DOUBLE(a[3]);
   int rc;
-  CALL(rc, p_norm_qmm(ptr(*x), ptr(*r), ptr(*nw), eps, ptr(h), ptr(nn), static_cast<const uint32_t*>(ptr(*w)), ptr(*s),
-                      ptr(*b), ptr(y), m, n, k, 64, 4, 1, silu ? QMM4_EPILOGUE_SILU_MUL : QMM4_EPILOGUE_NONE, st))
+  CALL(rc, p_norm_qmm(xp, rp, np, eps, hp, nnp, q.w, q.s, q.b, yp, m, n, k, 64, 4, 1,
+                      silu ? QMM4_EPILOGUE_SILU_MUL : QMM4_EPILOGUE_NONE, st))
   if (rc != 0) return PyLong_FromLong(rc);
   PyObject* out = PyTuple_New(3);
   if (!out) return nullptr;

@@ -86,3 +86,22 @@ def test_native_linear_follows_replaced_buffers():
     assert torch.equal(mod(x), quantized_matmul(x, *w2))
     mod.weight.data = weights(64, 256, seed=10)[0]
     assert torch.equal(mod(x), quantized_matmul(x, mod.weight, mod.scales, mod.biases))
+
+
+def test_native_raises_under_a_transform_of_its_outputs():
+    """Inside torch.func.grad new tensors are wrappers without storage: the calls raise, as their Python form does,
+    with the interpreter's lock held."""
+    w, s, b = weights(96, 256)
+    mod = QuantizedLinear.from_quantized(w, s, b)
+    install(torch.nn.ModuleList([mod]), verbose=False)
+    x, nw, w8 = rows(3, 256), rows(256), weights(33, 256, 8, 32)
+    calls = [lambda: quantized_matmul(x, w, s, b), lambda: quantized_matmul(x, *w8, group_size=32, bits=8),
+             lambda: mod(x), lambda: gate_up_silu(x, w, s, b), lambda: add_rms_norm_(x, x, nw, 1e-6),
+             lambda: add_rms_norm_qmm_(x, x, nw, 1e-6, w, s, b)]
+    for call in calls:
+        def inside(t):
+            with pytest.raises(RuntimeError, match="storage"):
+                call()
+            return (t * t).sum()
+        torch.func.grad(inside)(torch.ones(2, device=DEV))
+        assert all(torch.isfinite(t.float()).all() for t in torch.utils._pytree.tree_leaves(call()))
